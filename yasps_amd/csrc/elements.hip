@@ -462,25 +462,7 @@ __global__ void __launch_bounds__(64)
         for (int j = 0; j < 3; ++j)
           if (k < l || i <= j) M[upper_index<9>(3 * k + i, 3 * l + j)] = blk[i][j];
     }
-  double V[9][9];
-  jacobi_eigen_packed<9>(M, V);
-  double lam_c[9];
-#pragma unroll
-  for (int i = 0; i < 9; ++i) {
-    const double l = M[upper_index<9>(i, i)];
-    lam_c[i] = (l < 0.0) ? (prm.method == 1 ? -l : 0.0) : l;
-  }
-  // projected M' = V diag(lam_c) V^T (packed upper)
-  double Mp[kP];
-#pragma unroll
-  for (int i = 0; i < 9; ++i)
-#pragma unroll
-    for (int j = i; j < 9; ++j) {
-      double acc = 0.0;
-#pragma unroll
-      for (int k = 0; k < 9; ++k) acc += V[i][k] * lam_c[k] * V[j][k];
-      Mp[upper_index<9>(i, j)] = acc;
-    }
+  clamp_spectrum_packed<9>(M, prm.method);
   VertexSlots<4> vs;
   load_vertex_slots<KT>(SA, e, vs);
   scatter_hessian(SA, e, vs, [&](int a, int b, double out[3][3]) {
@@ -494,7 +476,7 @@ __global__ void __launch_bounds__(64)
 #pragma unroll
           for (int j = 0; j < 3; ++j) {
             const int r = 3 * k + i, c = 3 * l + j;
-            out[i][j] += w * Mp[r <= c ? upper_index<9>(r, c) : upper_index<9>(c, r)];
+            out[i][j] += w * M[r <= c ? upper_index<9>(r, c) : upper_index<9>(c, r)];
           }
       }
   });

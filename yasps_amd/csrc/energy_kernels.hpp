@@ -129,7 +129,7 @@ __device__ __forceinline__ uint32_t union_child(const UnionView& U, uint32_t v, 
 // ----------------------------------------------------------------- projection
 // hessianKernelHeader.pyx:79-252 for N >= 4: the packed-Schur PSD test on the element
 // Hessian; a failing matrix is replaced by V max(L, 0) V^T (method 2) or V |L| V^T
-// (method 1) from a cyclic Jacobi eigen-decomposition.
+// (method 1) from its eigen-decomposition (dense.hpp).
 template <int N>
 __device__ __forceinline__ void project_packed(double (&H)[N * (N + 1) / 2], uint32_t method) {
   double L[N * (N + 1) / 2];
@@ -138,32 +138,15 @@ __device__ __forceinline__ void project_packed(double (&H)[N * (N + 1) / 2], uin
 #pragma unroll
     for (int c = 0; c <= r; ++c) L[r * (r + 1) / 2 + c] = H[upper_index<N>(c, r)];
   if (psd_test_packed<N>(L)) return;
-  double V[N][N];
-  jacobi_eigen_packed<N>(H, V);
-  double lam[N];
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    const double l = H[upper_index<N>(i, i)];
-    lam[i] = (l < 0.0) ? (method == 1 ? -l : 0.0) : l;
-  }
-#pragma unroll
-  for (int i = 0; i < N; ++i)
-#pragma unroll
-    for (int j = i; j < N; ++j) {
-      double acc = 0.0;
-#pragma unroll
-      for (int k = 0; k < N; ++k) acc += V[i][k] * lam[k] * V[j][k];
-      H[upper_index<N>(i, j)] = acc;
-    }
+  clamp_spectrum_packed<N>(H, method);
 }
 
 // 4-vertex kinds whose energy depends on vertex differences only (barriers, dihedral
 // bending, SNH): their 12x12 Hessians annihilate the three translations, so a failing
 // Hessian is projected in the 9-dimensional complement, H = (U x I3) M (U x I3)^T with U
 // the orthonormal 4x3 basis orthogonal to (1,1,1,1): the same result as the 12x12
-// decomposition up to the rounding-level translation eigenvalues, on a 9x9 Jacobi
-// (0.42 of the rotations' work and 81 instead of 144 eigenvector registers). The PSD
-// test stays on the full 12x12 matrix, as the reference runs it.
+// decomposition up to the rounding-level translation eigenvalues, on a 9x9 matrix (0.42 of
+// the work and 81 instead of 144 eigenvector registers). The PSD test stays on the full 12x12 matrix, as the reference runs it.
 template <int ID>
 __host__ __device__ constexpr bool translation_free() {
   return ID == YSP_ENERGY_POINT_TRIANGLE || ID == YSP_ENERGY_EDGE_EDGE ||
@@ -205,25 +188,8 @@ __device__ __forceinline__ void project_translation_free(double (&H)[78], uint32
               acc += basis4(a, k) * basis4(b, l) * h12(3 * a + i, 3 * b + j);
           M[upper_index<9>(3 * k + i, 3 * l + j)] = acc;
         }
-  double V[9][9];
-  jacobi_eigen_packed<9>(M, V);
-  double lam[9];
-#pragma unroll
-  for (int i = 0; i < 9; ++i) {
-    const double l = M[upper_index<9>(i, i)];
-    lam[i] = (l < 0.0) ? (method == 1 ? -l : 0.0) : l;
-  }
-  double P[45];
-#pragma unroll
-  for (int i = 0; i < 9; ++i)
-#pragma unroll
-    for (int j = i; j < 9; ++j) {
-      double acc = 0.0;
-#pragma unroll
-      for (int k = 0; k < 9; ++k) acc += V[i][k] * lam[k] * V[j][k];
-      P[upper_index<9>(i, j)] = acc;
-    }
-  auto p9 = [&](int r, int c) { return r <= c ? P[upper_index<9>(r, c)] : P[upper_index<9>(c, r)]; };
+  clamp_spectrum_packed<9>(M, method);
+  auto p9 = [&](int r, int c) { return r <= c ? M[upper_index<9>(r, c)] : M[upper_index<9>(c, r)]; };
 #pragma unroll
   for (int a = 0; a < 4; ++a)
 #pragma unroll
