@@ -557,6 +557,43 @@ typedef struct ysp_upper_values {
   const double* dynamic_values;      /* of the dynamic part (NULL: none) */
 } ysp_upper_values;
 
+/* Tiled symmetric operator (no reference counterpart): the operator of a mirrored full
+ * block-CSR whose (row, column) entries do not repeat, laid out so that a block whose two
+ * rows share a tile of YSP_TILE_ROWS rows is stored once (see csrc/tiles.hpp). The PCG
+ * entry point ysp_pcg3_solve reads it with values_f32 = YSP_VALUES_TILED and values pointing
+ * to a host ysp_tiled_values; the products equal the mirrored copy's up to the order of each
+ * row's sum. Built in two steps:
+ * ysp_bsr3_tiles_layout orders the block rows (along a space-filling curve through points,
+ * [n] coordinates, 3 per block row; NULL: as they are) and returns the entry count (0: an
+ * operator with rows too long for tiles; synchronous); the caller then allocates entry and
+ * source [entries] and calls ysp_bsr3_tiles_entries. rows, lens [n / 3]; slice_start
+ * [YSP_TILE_SLICES(n / 3) + 1]; work [2 n / 3], kept between the two calls. ysp_bsr3_tiles_values
+ * gathers the values (9 per entry, 64 entries together; FP64 and/or FP32) from the upper
+ * block storage after each assembly. */
+#define YSP_VALUES_TILED 3
+#define YSP_TILE_ROWS 256
+#define YSP_TILE_SLICES(block_rows) \
+  (((block_rows) + YSP_TILE_ROWS - 1) / YSP_TILE_ROWS * (YSP_TILE_ROWS / 64))
+
+typedef struct ysp_tiled_values {
+  const uint32_t* rows;
+  const uint32_t* lens;
+  const uint32_t* slice_start;
+  const uint32_t* entry;
+  uint32_t entries;
+  const void* values;
+  int32_t values_f32;
+} ysp_tiled_values;
+
+int ysp_bsr3_tiles_layout(const uint32_t* row_ptr, const uint32_t* col, uint32_t nnz, uint32_t n,
+                          const double* points, uint32_t* rows, uint32_t* lens,
+                          uint32_t* slice_start, uint32_t* work, uint32_t* entries, void* stream);
+int ysp_bsr3_tiles_entries(const uint32_t* row_ptr, const uint32_t* col, const uint32_t* src,
+                           uint32_t n, const uint32_t* rows, const uint32_t* slice_start,
+                           const uint32_t* work, uint32_t* entry, uint32_t* source, void* stream);
+int ysp_bsr3_tiles_values(const double* static_values, const uint32_t* source, uint32_t entries,
+                          double* out64, float* out32, void* stream);
+
 /* out[i] = (float) in[i] (FP32 copies of FP64 device arrays, e.g. inverse blocks). */
 int ysp_cast_f32(const double* in, float* out, uint64_t n, void* stream);
 

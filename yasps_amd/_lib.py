@@ -61,13 +61,21 @@ class CoordDim(C.Structure):
                 ("w", C.c_uint16), ("placeholder", C.c_uint32)]
 
 
-VALUES_F64, VALUES_F32, VALUES_UPPER = 0, 1, 2
+VALUES_F64, VALUES_F32, VALUES_UPPER, VALUES_TILED = 0, 1, 2, 3
+TILE_ROWS = 256
 
 
 class UpperValues(C.Structure):
     """ysp_upper_values: the upper block storage read through each entry's source word."""
     _fields_ = [("src", C.c_void_p), ("src_64", C.c_int32), ("static_values", C.c_void_p),
                 ("dynamic_values", C.c_void_p)]
+
+
+class TiledValues(C.Structure):
+    """ysp_tiled_values: the tiled symmetric operator of the PCG product."""
+    _fields_ = [("rows", C.c_void_p), ("lens", C.c_void_p), ("slice_start", C.c_void_p),
+                ("entry", C.c_void_p), ("entries", C.c_uint32), ("values", C.c_void_p),
+                ("values_f32", C.c_int32)]
 
 
 class PcgStats(C.Structure):
@@ -148,6 +156,9 @@ SIGNATURES = {
     "ysp_gather_gradient3": (C.c_int, [P, P, P, U32, P, P]),
     "ysp_bsr3_build": (C.c_int, [P, U32, P, U32, U32, P, P, P, U32, C.POINTER(U32), P]),
     "ysp_bsr3_gather_values": (C.c_int, [P, P, P, U32, P, P, P]),
+    "ysp_bsr3_tiles_layout": (C.c_int, [P, P, U32, U32, P, P, P, P, P, C.POINTER(U32), P]),
+    "ysp_bsr3_tiles_entries": (C.c_int, [P, P, P, U32, P, P, P, P, P, P]),
+    "ysp_bsr3_tiles_values": (C.c_int, [P, P, U32, P, P, P]),
     "ysp_cast_f32": (C.c_int, [P, P, C.c_uint64, P]),
     "ysp_bsr3_spmv": (C.c_int, [P, P, P, I32, U32, U32, P, P, P]),
     "ysp_bsr3_refine": (C.c_int, [P, P, P, I32, U32, U32, P, P, P, P, C.POINTER(D), C.POINTER(D),

@@ -12,6 +12,7 @@
 #include "common.hpp"
 #include "dense.hpp"
 #include "mas.hpp"
+#include "tiles.hpp"
 #include "values.hpp"
 
 #include <cmath>
@@ -19,6 +20,7 @@
 #include <hipcub/hipcub.hpp>
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 namespace ysp {
@@ -493,6 +495,245 @@ __global__ void __launch_bounds__(kB)
   }
 }
 
+// One thread's share of a tile's product (tiles.hpp): y of its row in registers, what the
+// tile's other rows owe it in ys (LDS, FP64 atomics on distinct words: consecutive lanes
+// hold consecutive positions). kTileTpr threads share a row, every kTileTpr-th entry each.
+// Two groups of kTileU entries are in registers at a time: the first two are asked for
+// before the tile's part of z has arrived (their addresses need only the row's length),
+// later ones while a group is worked on.
+constexpr int kTileTpr = 2;
+constexpr int kTileU = 1;
+constexpr int kTileThreads = kTileRows * kTileTpr;
+
+template <typename VT>
+struct TileGroup {
+  uint32_t w[kTileU];
+  VT b[kTileU][9];
+  __device__ __forceinline__ void load(const Tiled<VT>& T, uint32_t base, uint32_t j, uint32_t len) {
+#pragma unroll
+    for (int u = 0; u < kTileU; ++u) {
+      const uint32_t ju = j + u * kTileTpr;
+      if (ju >= len) continue;
+      const uint32_t k = base + 64 * ju;
+      w[u] = T.t.entry[k];
+      const VT* v = T.v + tile_value(k);
+#pragma unroll
+      for (int i = 0; i < 9; ++i) b[u][i] = v[64 * i];
+    }
+  }
+};
+
+template <typename VT>
+struct TileRow {
+  uint32_t len = 0, base = 0, self = 0;
+  double x[3], y[3] = {0.0, 0.0, 0.0};
+
+  __device__ __forceinline__ void open(const Tiled<VT>& T, uint32_t pos, uint32_t nv) {
+    self = pos % kTileRows;
+    if (pos < nv) {
+      len = T.t.lens[pos];
+      base = T.t.slice_start[pos / 64] + pos % 64;
+    }
+  }
+
+  __device__ __forceinline__ void apply(const TileGroup<VT>& G, uint32_t j,
+                                        const double* __restrict__ z, const double* xs, double* ys) {
+    double c[kTileU][3];
+#pragma unroll
+    for (int u = 0; u < kTileU; ++u) {
+      if (j + u * kTileTpr >= len) continue;
+      const uint32_t w = G.w[u];
+      if (w & kTileCut) {
+        const double* zc = z + 3 * static_cast<size_t>(w & ~kTileCut);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) c[u][i] = zc[i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) c[u][i] = xs[3 * w + i];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kTileU; ++u) {
+      if (j + u * kTileTpr >= len) continue;
+      double b[9];
+#pragma unroll
+      for (int i = 0; i < 9; ++i) b[i] = static_cast<double>(G.b[u][i]);
+      block_fma(b, c[u][0], c[u][1], c[u][2], y[0], y[1], y[2]);
+      const uint32_t w = G.w[u];
+      if (w >= kTileCut || w == self) continue;
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        atomic_add_f64(ys + 3 * w + i, fma(b[i], x[0], fma(b[3 + i], x[1], b[6 + i] * x[2])));
+    }
+  }
+
+  // The groups from j = share on, the first two already asked for; y goes to ys.
+  __device__ __forceinline__ void product(const Tiled<VT>& T, uint32_t share, TileGroup<VT>& A,
+                                          TileGroup<VT>& B, const double* __restrict__ z,
+                                          const double* xs, double* ys) {
+    constexpr uint32_t kStep = kTileU * kTileTpr;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) x[i] = xs[3 * self + i];
+    for (uint32_t j = share; j < len; j += 2 * kStep) {
+      apply(A, j, z, xs, ys);
+      A.load(T, base, j + 2 * kStep, len);
+      if (j + kStep >= len) break;
+      apply(B, j + kStep, z, xs, ys);
+      B.load(T, base, j + 3 * kStep, len);
+    }
+    if (len)
+#pragma unroll
+      for (int i = 0; i < 3; ++i) atomic_add_f64(ys + 3 * self + i, y[i]);
+  }
+};
+
+// pcg3_spmv_kernel over the tiled operator (same recurrence, tests and scalar state), z, p
+// and q in tile order (in the caller's order their scattered 24-byte pieces were 40% of the
+// L1 accesses: 22.1 against 18.4 us). Bound by the bytes: 48^3-cell cube 1.12M entries of 76
+// bytes and five vectors, 100 MB in 17.6 us, 5.7 TB/s where plain reads of resident data
+// reach 6.8 (mirrored 148 MB in 23.8 us); 64^3 cells 40.7 us (upper storage in place 45.3).
+// 512 threads at 100 VGPRs put two tiles on a compute unit; one entry per thread and group
+// measured 17.6, two 18.6, more wavefronts by spilling 30 us; tiles of 512 rows 17.0 / 44.9
+// us, of 128 rows 19.8 / 41.7 (48^3 / 64^3 cells).
+template <typename VT>
+__global__ void __launch_bounds__(kTileThreads, 4)
+    pcg3_tiled_kernel(Tiled<VT> T, uint32_t nv, const double* __restrict__ z,
+                      double* __restrict__ p, double* __restrict__ q, double* __restrict__ st,
+                      int k, int reverse) {
+  const uint32_t blk = xcd_swizzle(blockIdx.x, gridDim.x);
+  const uint32_t tile = reverse ? gridDim.x - 1 - blk : blk;
+  const uint32_t share = threadIdx.x / kTileRows;
+  const int cur = k % 3, prev = (k + 2) % 3, prev2 = (k + 1) % 3;
+  __shared__ double xs[3 * kTileRows], ys[3 * kTileRows], lds[kTileThreads / 64];
+  __shared__ double head[4];
+  TileRow<VT> R;
+  R.open(T, tile * kTileRows + threadIdx.x % kTileRows, nv);
+  // the state, the tile's part of z, p and q and the first entries together
+  LoopState L;
+  L.issue(st, SET_RZ + prev, SET_RR + prev, SET_RZ + prev2);
+  constexpr int kPer = (3 * kTileRows + kTileThreads - 1) / kTileThreads;
+  const uint32_t first = 3 * kTileRows * tile, live = min(3 * kTileRows, 3 * nv - first);
+  double zt[kPer], pt[kPer], qt[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const uint32_t t = threadIdx.x + i * kTileThreads;
+    zt[i] = pt[i] = qt[i] = 0.0;
+    if (t < live) {
+      zt[i] = z[first + t];
+      if (k > 1) {
+        pt[i] = p[first + t];
+        qt[i] = q[first + t];
+      }
+    }
+  }
+  TileGroup<VT> A, B;
+  A.load(T, R.base, share, R.len);
+  B.load(T, R.base, share + kTileU * kTileTpr, R.len);
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const uint32_t t = threadIdx.x + i * kTileThreads;
+    if (t < 3 * kTileRows) {
+      xs[t] = zt[i];
+      ys[t] = 0.0;
+    }
+  }
+  if (L.finish(head)) return;
+  const double rz1 = L.a, rr1 = L.b, rz2 = L.c;
+  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+  double beta = 0.0;
+  if (k > 1) {
+    if (!isfinite(rz1) || rz1 < 0.0 || !isfinite(rz2) || !(rz2 > 0.0)) {
+      if (lead) {
+        st[S_STATUS] = -1.0;
+        st[S_ITER] = k - 1;
+      }
+      return;
+    }
+    if ((L.mode == 0.0 ? rz1 : rr1) <= L.thr) {
+      if (lead) {
+        st[S_STATUS] = 1.0;
+        st[S_ITER] = k - 1;
+        st[S_FINAL_RZ] = rz1;
+        st[S_FINAL_RR] = rr1;
+      }
+      return;
+    }
+    beta = rz1 / rz2;
+  }
+  if (lead) {
+    st[S_FINAL_RZ] = rz1;
+    st[S_FINAL_RR] = rr1;
+    st[S_CUR_ITER] = k - 1;
+  }
+  R.product(T, share, A, B, z, xs, ys);
+  __syncthreads();
+  double pap = 0.0;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const uint32_t t = threadIdx.x + i * kTileThreads;
+    if (t >= live) continue;
+    // first direction (beta = 0, p and q taken as 0): p = z, q = A z
+    const double pn = fma(pt[i], beta, zt[i]), qn = fma(qt[i], beta, ys[t]);
+    p[first + t] = pn;
+    q[first + t] = qn;
+    pap = fma(pn, qn, pap);
+  }
+  pap = block_sum<kTileThreads>(pap, lds);
+  if (threadIdx.x == 0) atomic_add_f64(slot_ptr(st, SET_PAP + cur), pap);
+}
+
+// y = A x over the tiled operator, x and y in tile order.
+template <typename VT>
+__global__ void __launch_bounds__(kTileThreads, 4)
+    tiled_spmv_kernel(Tiled<VT> T, uint32_t nv, const double* __restrict__ x,
+                      double* __restrict__ y) {
+  const uint32_t tile = xcd_swizzle(blockIdx.x, gridDim.x);
+  const uint32_t share = threadIdx.x / kTileRows;
+  __shared__ double xs[3 * kTileRows], ys[3 * kTileRows];
+  TileRow<VT> R;
+  R.open(T, tile * kTileRows + threadIdx.x % kTileRows, nv);
+  const uint32_t first = 3 * kTileRows * tile, live = min(3 * kTileRows, 3 * nv - first);
+  TileGroup<VT> A, B;
+  A.load(T, R.base, share, R.len);
+  B.load(T, R.base, share + kTileU * kTileTpr, R.len);
+  for (uint32_t t = threadIdx.x; t < 3 * kTileRows; t += kTileThreads) {
+    xs[t] = t < live ? x[first + t] : 0.0;
+    ys[t] = 0.0;
+  }
+  __syncthreads();
+  R.product(T, share, A, B, x, xs, ys);
+  __syncthreads();
+  for (uint32_t t = threadIdx.x; t < live; t += kTileThreads) y[first + t] = ys[t];
+}
+
+// Into tile order (b, x0 and the 3x3 inverse blocks) and, for the solution, back.
+template <typename MT>
+__global__ void __launch_bounds__(kB)
+    tile_order_kernel(const uint32_t* __restrict__ rows, uint32_t nv, const double* __restrict__ b,
+                      const double* __restrict__ x0, const MT* __restrict__ minv,
+                      double* __restrict__ bt, double* __restrict__ xt, MT* __restrict__ mt) {
+  const uint32_t i = blockIdx.x * kB + threadIdx.x;     // one inverse entry per thread
+  if (i >= 9 * nv) return;
+  const uint32_t pos = i / 9, e = i % 9, r = rows[pos];
+  mt[i] = minv[9 * static_cast<size_t>(r) + e];
+  if (e < 3) {
+    bt[3 * static_cast<size_t>(pos) + e] = b[3 * static_cast<size_t>(r) + e];
+    if (x0) xt[3 * static_cast<size_t>(pos) + e] = x0[3 * static_cast<size_t>(r) + e];
+  }
+}
+
+__global__ void __launch_bounds__(kB)
+    tile_unorder_kernel(const uint32_t* __restrict__ rows, uint32_t n, const double* __restrict__ xt,
+                        double* __restrict__ x) {
+  const uint32_t i = blockIdx.x * kB + threadIdx.x;
+  if (i < n) x[3 * static_cast<size_t>(rows[i / 3]) + i % 3] = xt[i];
+}
+
+template <typename Src>
+struct is_tiled : std::false_type {};
+template <typename VT>
+struct is_tiled<Tiled<VT>> : std::true_type {};
+
 // Iteration k, kernel 2: alpha, x += alpha p, r -= alpha q, z = M^-1 r, r.z and r.r.
 // One thread per scalar (coalesced vector traffic); a workgroup of 192 threads holds 64
 // whole vertices, whose residual 3-vectors meet in LDS for the block-Jacobi product.
@@ -604,9 +845,14 @@ long predict_more(double it_a, double val_a, double it_b, double val_b, double t
 template <typename Src>
 void launch_full_spmv(const uint32_t* row_ptr, const uint32_t* col, const Src& vals, uint32_t nbr,
                       const double* x, double* y, hipStream_t s) {
-  const unsigned rows_per_block = kB / kG;
-  hipLaunchKernelGGL(bsr3_full_spmv_kernel<Src>, dim3(grid_for(nbr, rows_per_block)), dim3(kB), 0,
-                     s, row_ptr, col, vals, nbr, x, y);
+  if constexpr (is_tiled<Src>::value) {
+    hipLaunchKernelGGL(tiled_spmv_kernel, dim3(grid_for(nbr, kTileRows)), dim3(kTileThreads), 0, s,
+                       vals, nbr, x, y);
+  } else {
+    const unsigned rows_per_block = kB / kG;
+    hipLaunchKernelGGL(bsr3_full_spmv_kernel<Src>, dim3(grid_for(nbr, rows_per_block)), dim3(kB), 0,
+                       s, row_ptr, col, vals, nbr, x, y);
+  }
 }
 
 }  // namespace
@@ -1032,6 +1278,24 @@ int pcg3_run(uint32_t max_iterations, double threshold, int32_t mode, const uint
                        static_cast<uint32_t>(kStateDoubles));
   else
     YSP_CHECK(hipMemsetAsync(st, 0, kStateDoubles * sizeof(double), s));
+  // The tiled operator's loop runs in tile order on copies of b, x0 and the inverse blocks
+  // (library scratch, 7 n values); the solution is put back at the end.
+  double* const solution = x;
+  if constexpr (is_tiled<Src>::value) {
+    if (!minv || n > 0xffffffffu / 3) {
+      ysp_set_error(__FILE__, __LINE__, "PCG: tiles need inverse blocks and fewer than 2^32 / 3 unknowns");
+      return YSP_ERR_ARG;
+    }
+    double* tv = static_cast<double*>(ysp::scratch(128, sizeof(double) * 3 * n));
+    MT* tm = static_cast<MT*>(ysp::scratch(129, sizeof(MT) * 3 * n));
+    if (!tv || !tm) return YSP_ERR_HIP;
+    hipLaunchKernelGGL(tile_order_kernel<MT>, dim3(grid_for(9 * static_cast<size_t>(nv), kB)),
+                       dim3(kB), 0, s, vals.t.rows, nv, rhs, x0, minv, tv, tv + n, tm);
+    rhs = tv;
+    x = tv + 2 * static_cast<size_t>(n);
+    if (x0) x0 = tv + n;
+    minv = tm;
+  }
   const double* ax0 = nullptr;
   if (x0) {
     launch_full_spmv(row_ptr, col, vals, nv, x0, q, s);
@@ -1055,8 +1319,8 @@ int pcg3_run(uint32_t max_iterations, double threshold, int32_t mode, const uint
   uint32_t* long_slot = nullptr;
   double* ylong = nullptr;
   uint32_t* chunk_start = nullptr;
-  if (no_alloc) {
-    // every row through the product kernel, uniform chunks
+  if (no_alloc || is_tiled<Src>::value) {
+    // every row through the product kernel, uniform chunks (or the operator's tiles)
   } else if (cache.row_ptr == row_ptr && cache.nv == nv && cache.nnz == nnz) {
     num_long = cache.num_long;
     num_chunks = cache.num_chunks;
@@ -1122,12 +1386,17 @@ int pcg3_run(uint32_t max_iterations, double threshold, int32_t mode, const uint
   const uint32_t end = max_iterations + 1;
   auto launch_pass = [&](uint32_t it) -> int {
     const int reverse = static_cast<int>(it & 1u);
-    if (num_long)
-      hipLaunchKernelGGL(pcg3_long_rows_kernel<Src>, dim3(num_long), bl, 0, s, row_ptr, col, vals,
-                         long_rows, z, ylong, st, reverse);
-    hipLaunchKernelGGL(pcg3_spmv_kernel<Src>, sg, bl, 0, s, row_ptr, col, vals, nv, z, pa, q,
-                       st, static_cast<int>(it), rows_per_wg, long_slot, ylong, chunk_start,
-                       reverse);
+    if constexpr (is_tiled<Src>::value) {
+      hipLaunchKernelGGL(pcg3_tiled_kernel, dim3(grid_for(nv, kTileRows)), dim3(kTileThreads), 0, s,
+                         vals, nv, z, pa, q, st, static_cast<int>(it), reverse);
+    } else {
+      if (num_long)
+        hipLaunchKernelGGL(pcg3_long_rows_kernel<Src>, dim3(num_long), bl, 0, s, row_ptr, col, vals,
+                           long_rows, z, ylong, st, reverse);
+      hipLaunchKernelGGL(pcg3_spmv_kernel<Src>, sg, bl, 0, s, row_ptr, col, vals, nv, z, pa, q,
+                         st, static_cast<int>(it), rows_per_wg, long_slot, ylong, chunk_start,
+                         reverse);
+    }
     if (it <= max_iterations) {
       hipLaunchKernelGGL(pcg3_update_kernel<MT>, ug, dim3(kUB), 0, s, minv, x, r, pa, q, z, n, st,
                          static_cast<int>(it));
@@ -1140,6 +1409,11 @@ int pcg3_run(uint32_t max_iterations, double threshold, int32_t mode, const uint
     return YSP_OK;
   };
   auto finish = [&]() -> int {
+    if constexpr (is_tiled<Src>::value) {
+      hipLaunchKernelGGL(tile_unorder_kernel, dim3(grid_for(n, kB)), bl, 0, s, vals.t.rows, n, x,
+                         solution);
+      YSP_CHECK_LAUNCH();
+    }
     double fin[S_HEADER];
     YSP_CHECK(hipMemcpyAsync(fin, st, sizeof(fin), hipMemcpyDeviceToHost, s));
     YSP_CHECK(hipStreamSynchronize(s));
@@ -1254,6 +1528,20 @@ int pcg3_run(uint32_t max_iterations, double threshold, int32_t mode, const uint
 }  // namespace
 
 namespace {
+// with_values, and the tiled operator (which only the block-Jacobi loop reads).
+template <typename F>
+int with_pcg_values(const void* values, int32_t format, uint32_t nnz, const char* who, F&& f) {
+  if (format != YSP_VALUES_TILED) return with_values(values, format, nnz, who, f);
+  const ysp_tiled_values* t = static_cast<const ysp_tiled_values*>(values);
+  if (!t || !t->rows || !t->lens || !t->slice_start || !t->entry || !t->values) {
+    ysp_set_error(__FILE__, __LINE__, who);
+    return YSP_ERR_ARG;
+  }
+  const TiledView v{t->rows, t->lens, t->slice_start, t->entry, t->entries};
+  if (t->values_f32) return f(Tiled<float>{v, static_cast<const float*>(t->values)});
+  return f(Tiled<double>{v, static_cast<const double*>(t->values)});
+}
+
 // Dispatch on the value source (values.hpp) and the inverse type (FP64 / FP32).
 int pcg3_dispatch(uint32_t max_iterations, double threshold, int32_t threshold_mode,
                   const uint32_t* row_ptr, const uint32_t* col, const void* values,
@@ -1261,7 +1549,7 @@ int pcg3_dispatch(uint32_t max_iterations, double threshold, int32_t threshold_m
                   int32_t inverse_f32, const double* rhs, uint32_t n, double* solution,
                   const double* x0, double* work, double* cg_scalars, ysp_pcg_stats* stats,
                   hipStream_t s, bool no_alloc) {
-  return with_values(values, value_format, nnz, "PCG: bad value source", [&](auto vals) {
+  auto run = [&](auto vals) {
     if (inverse_f32)
       return pcg3_run(max_iterations, threshold, threshold_mode, row_ptr, col, vals, nnz,
                       static_cast<const float*>(diagonal_inverse), nullptr, rhs, n, solution, x0,
@@ -1269,7 +1557,10 @@ int pcg3_dispatch(uint32_t max_iterations, double threshold, int32_t threshold_m
     return pcg3_run(max_iterations, threshold, threshold_mode, row_ptr, col, vals, nnz,
                     static_cast<const double*>(diagonal_inverse), nullptr, rhs, n, solution, x0,
                     work, cg_scalars, stats, s, no_alloc);
-  });
+  };
+  const char* who = "PCG: bad value source";
+  return no_alloc ? with_values(values, value_format, nnz, who, run)
+                  : with_pcg_values(values, value_format, nnz, who, run);
 }
 }  // namespace
 

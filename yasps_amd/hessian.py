@@ -185,6 +185,21 @@ _STRUCTURE_VERSIONS = itertools.count(1)
 
 
 @dataclass
+class Tiles:
+    """Tiled symmetric form of a full block-CSR (``ysp_bsr3_tiles_layout``) and its values."""
+    rows: object
+    lens: object
+    slice_start: object
+    entry: object
+    source: object
+    entries: int
+    v64: object = None
+    v32: object = None
+    valid64: bool = False        # v64 / v32 hold the current values
+    valid32: bool = False
+
+
+@dataclass
 class FullBsr:
     """Mirrored full 3x3 block-CSR of the current layout (the solve loop's operator)."""
     key: tuple
@@ -195,6 +210,7 @@ class FullBsr:
     nnz: int
     v64: object = None
     v32: object = None
+    tiles: Optional[Tiles] = None
     v32_valid: bool = False      # v32 holds the current values
     # changes only when the structure does (a rebuild onto the same pairs keeps it)
     version: int = field(default_factory=lambda: next(_STRUCTURE_VERSIONS))
@@ -243,6 +259,7 @@ class hessian:
         # the mirrored copy would not stay in the Infinity Cache), "mirrored" or "upper"
         self.value_source = "auto"
         self._upper = None
+        self._tiled = None
         self.use_staging = True
         self._grad_offsets = None
 
@@ -474,6 +491,77 @@ class hessian:
                                             self.rows, dev.ptr(self.gradient.value), s),
                    "ysp_gather_gradient3")
 
+    # --------------------------------------------------------------- tiles
+    # Mirrored values below this many bytes (FP64) stay in the XCDs' L2 caches (32 MB in
+    # all) and the plain product is bound by latency, not bytes. Newton solve, tiled against
+    # plain: 960 us plain, 1,093 tiled at 15 MB; 1,261 / 1,314 at 24 MB; 1,491 / 1,460 at
+    # 33 MB; 2,146 / 1,972 at 51 MB (FP32 values with FP64 refinement cross at the same size:
+    # 1,307 / 1,350 at 24 MB, 1,551 / 1,476 at 33 MB).
+    TILE_VALUE_BYTES = 28 << 20
+
+    def _build_tiles(self, f: FullBsr):
+        """Tiles of a static operator large enough to gain from them, along a curve through
+        the targets' values (a mesh's positions)."""
+        if self.dynamic_terms or 72 * f.nnz < self.TILE_VALUE_BYTES:
+            return
+        lib = _lib.load()
+        t = dev.torch()
+        s = dev.stream()
+        points = [w.value.reshape(-1) for w in self.wrt]
+        points = points[0] if len(points) == 1 else t.cat(points)
+        if points.numel() != self.rows or points.dtype != t.float64:
+            return
+        points = points.contiguous()
+        nv = f.nbr
+        slices = (nv + _lib.TILE_ROWS - 1) // _lib.TILE_ROWS * (_lib.TILE_ROWS // 64)
+        rows, lens = dev.empty(nv, "uint32"), dev.empty(nv, "uint32")
+        slice_start = dev.empty(slices + 1, "uint32")
+        work = dev.empty(2 * nv, "uint32")
+        count = C.c_uint32(0)
+        _lib.check(lib.ysp_bsr3_tiles_layout(
+            dev.ptr(f.row_ptr), dev.ptr(f.col), f.nnz, self.rows, dev.ptr(points), dev.ptr(rows),
+            dev.ptr(lens), dev.ptr(slice_start), dev.ptr(work), C.byref(count), s),
+            "ysp_bsr3_tiles_layout")
+        n = count.value
+        if n == 0 or n > 0.9 * f.nnz:     # long rows, or points that tell nothing of the mesh
+            return
+        entry, source = dev.empty(n, "uint32"), dev.empty(n, "uint32")
+        _lib.check(lib.ysp_bsr3_tiles_entries(
+            dev.ptr(f.row_ptr), dev.ptr(f.col), dev.ptr(f.src), self.rows, dev.ptr(rows),
+            dev.ptr(slice_start), dev.ptr(work), dev.ptr(entry), dev.ptr(source), s),
+            "ysp_bsr3_tiles_entries")
+        f.tiles = Tiles(rows, lens, slice_start, entry, source, n)
+
+    def pcg_values(self, f32: bool = False):
+        """(pointer, format) of the operator values for the PCG entry points: the tiled
+        symmetric operator where the layout has one (``YSP_VALUES_TILED``), else
+        ``solve_values`` (the mirrored FP32 copy with f32)."""
+        f = self.operator
+        tl = f.tiles if f is not None and self.value_source == "auto" else None
+        if tl is None:
+            return (dev.ptr(self.full_values_f32()), _lib.VALUES_F32) if f32 else self.solve_values()
+        lib = _lib.load()
+        if f32:
+            if tl.v32 is None:
+                tl.v32 = dev.empty(9 * tl.entries, "float32")
+            if not tl.valid32:
+                _lib.check(lib.ysp_bsr3_tiles_values(dev.ptr(self.static.values), dev.ptr(tl.source),
+                                                     tl.entries, None, dev.ptr(tl.v32), dev.stream()),
+                           "ysp_bsr3_tiles_values")
+                tl.valid32 = True
+        else:
+            if tl.v64 is None:
+                tl.v64 = dev.empty(9 * tl.entries, "float64")
+            if not tl.valid64:
+                _lib.check(lib.ysp_bsr3_tiles_values(dev.ptr(self.static.values), dev.ptr(tl.source),
+                                                     tl.entries, dev.ptr(tl.v64), None, dev.stream()),
+                           "ysp_bsr3_tiles_values")
+                tl.valid64 = True
+        self._tiled = _lib.TiledValues(dev.ptr(tl.rows), dev.ptr(tl.lens), dev.ptr(tl.slice_start),
+                                       dev.ptr(tl.entry), tl.entries,
+                                       dev.ptr(tl.v32 if f32 else tl.v64), int(f32))
+        return C.addressof(self._tiled), _lib.VALUES_TILED
+
     # --------------------------------------------------------------- full block-CSR
     @property
     def all_3x3(self) -> bool:
@@ -552,7 +640,10 @@ class hessian:
                 self.full.key = key
             else:
                 self.full = new
+                self._build_tiles(new)
         f = self.full
+        if f.tiles is not None:
+            f.tiles.valid64 = f.tiles.valid32 = False
         stride = (f.nnz + 63) // 64 * 64
         if f.v64 is None or f.v64.numel() != 9 * stride:
             f.v64 = dev.empty(9 * stride, "float64")

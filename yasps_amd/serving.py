@@ -81,6 +81,7 @@ class _Slot:
         hs = self.scene.minimizer.activeHessian
         if hs.full is None:
             raise RuntimeError("serving needs the 3x3 full block-CSR path")
+        hs.full.tiles = None        # the batched PCG reads the mirrored copy
         self.hs = hs
         m = hs.rows
         self.solution = dev.zeros(m, "float64")

@@ -99,7 +99,7 @@ class jacobianPCGSolver:
             return self._solve_mixed(h, right_hand_side, n, tolerance, maxIterations, t0, t1, t2)
         if h.full is not None:
             f = h.full
-            vals, fmt = h.solve_values()
+            vals, fmt = h.pcg_values()
             rc = lib.ysp_pcg3_solve(
                 int(maxIterations), float(tolerance), _MODES[self.threshold_mode],
                 dev.ptr(f.row_ptr), dev.ptr(f.col), vals, fmt, f.nnz,
@@ -152,9 +152,9 @@ class jacobianPCGSolver:
         lib = _lib.load()
         s = dev.stream()
         f = h.operator
-        v32 = h.full_values_f32()
         stats = _lib.PcgStats()
         if h.full is None:
+            v32 = h.full_values_f32()
             # affine-body layout: the split operator in FP32, the reference's block-Jacobi
             # (9 x 9 inverse blocks for the affine matrices) kept in FP64
             counts = [w.numInstances for w in h.wrt]
@@ -178,9 +178,11 @@ class jacobianPCGSolver:
             _lib.check(lib.ysp_cast_f32(dev.ptr(h.diagonal_blocks_inverse), dev.ptr(self._minv32),
                                         nd, s), "ysp_cast_f32")
 
+            vals, fmt = h.pcg_values(f32=True)
+
             def inner(r, d, tol_in, max_it):
                 rc = lib.ysp_pcg3_solve(int(max_it), float(tol_in), 1, dev.ptr(f.row_ptr),
-                                        dev.ptr(f.col), dev.ptr(v32), 1, f.nnz, dev.ptr(self._minv32),
+                                        dev.ptr(f.col), vals, fmt, f.nnz, dev.ptr(self._minv32),
                                         1, dev.ptr(r), n, dev.ptr(d), None, 1, dev.ptr(self.__work),
                                         dev.ptr(self.__scalars), C.byref(stats), s)
                 _lib.check(rc, "ysp_pcg3_solve")
