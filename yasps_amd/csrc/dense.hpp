@@ -261,14 +261,14 @@ __device__ __forceinline__ void sym_eigen_packed(double (&a)[N * (N + 1) / 2], d
   for (int i = 0; i < N; ++i) d[i] = __builtin_amdgcn_ldexp(d[i], ex);
 }
 
-// The projection of hessianKernelHeader.pyx:143-252 on a packed upper triangle: negative
-// eigenvalues become 0 (method 2) or their absolute value (method 1).
-template <int N>
-__device__ __forceinline__ void clamp_spectrum_packed(double (&a)[N * (N + 1) / 2], uint32_t method) {
+// a = V diag(f(d)) V^T for the eigen-decomposition a = V diag(d) V^T of a packed upper
+// triangle.
+template <int N, typename F>
+__device__ __forceinline__ void map_spectrum_packed(double (&a)[N * (N + 1) / 2], F f) {
   double d[N], V[N][N];
   sym_eigen_packed<N>(a, d, V);
 #pragma unroll
-  for (int i = 0; i < N; ++i) d[i] = d[i] < 0.0 ? (method == 1 ? -d[i] : 0.0) : d[i];
+  for (int i = 0; i < N; ++i) d[i] = f(d[i]);
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     double t[N];
@@ -282,6 +282,17 @@ __device__ __forceinline__ void clamp_spectrum_packed(double (&a)[N * (N + 1) / 
       a[upper_index<N>(i, j)] = acc;
     }
   }
+}
+
+// The projection of hessianKernelHeader.pyx:143-252: negative eigenvalues become 0 (method
+// 2) or their absolute value (method 1); and what it adds to the matrix.
+template <int N>
+__device__ __forceinline__ void clamp_spectrum_packed(double (&a)[N * (N + 1) / 2], uint32_t method) {
+  map_spectrum_packed<N>(a, [=](double d) { return d < 0.0 ? (method == 1 ? -d : 0.0) : d; });
+}
+template <int N>
+__device__ __forceinline__ void clamp_change_packed(double (&a)[N * (N + 1) / 2], uint32_t method) {
+  map_spectrum_packed<N>(a, [=](double d) { return d < 0.0 ? (method == 1 ? -2.0 * d : -d) : 0.0; });
 }
 
 }  // namespace ysp

@@ -128,25 +128,37 @@ __device__ __forceinline__ uint32_t union_child(const UnionView& U, uint32_t v, 
 
 // ----------------------------------------------------------------- projection
 // hessianKernelHeader.pyx:79-252 for N >= 4: the packed-Schur PSD test on the element
-// Hessian; a failing matrix is replaced by V max(L, 0) V^T (method 2) or V |L| V^T
-// (method 1) from its eigen-decomposition (dense.hpp).
+// Hessian; a failing matrix H becomes V max(L, 0) V^T (method 2) or V |L| V^T (method 1),
+// formed as H plus the change of its negative eigenvalues (dense.hpp), so that what the
+// projection leaves alone keeps its bits.
 template <int N>
-__device__ __forceinline__ void project_packed(double (&H)[N * (N + 1) / 2], uint32_t method) {
+__device__ __forceinline__ bool is_psd(const double (&H)[N * (N + 1) / 2]) {
   double L[N * (N + 1) / 2];
 #pragma unroll
   for (int r = 0; r < N; ++r)
 #pragma unroll
     for (int c = 0; c <= r; ++c) L[r * (r + 1) / 2 + c] = H[upper_index<N>(c, r)];
-  if (psd_test_packed<N>(L)) return;
-  clamp_spectrum_packed<N>(H, method);
+  return psd_test_packed<N>(L);
+}
+
+template <int N>
+__device__ __forceinline__ void project_packed(double (&H)[N * (N + 1) / 2], uint32_t method) {
+  if (is_psd<N>(H)) return;
+  double D[N * (N + 1) / 2];
+#pragma unroll
+  for (int i = 0; i < N * (N + 1) / 2; ++i) D[i] = H[i];
+  clamp_change_packed<N>(D, method);
+#pragma unroll
+  for (int i = 0; i < N * (N + 1) / 2; ++i) H[i] += D[i];
 }
 
 // 4-vertex kinds whose energy depends on vertex differences only (barriers, dihedral
 // bending, SNH): their 12x12 Hessians annihilate the three translations, so a failing
-// Hessian is projected in the 9-dimensional complement, H = (U x I3) M (U x I3)^T with U
+// Hessian is projected in the 9-dimensional complement, M = (U x I3)^T H (U x I3) with U
 // the orthonormal 4x3 basis orthogonal to (1,1,1,1): the same result as the 12x12
 // decomposition up to the rounding-level translation eigenvalues, on a 9x9 matrix (0.42 of
-// the work and 81 instead of 144 eigenvector registers). The PSD test stays on the full 12x12 matrix, as the reference runs it.
+// the work and 81 instead of 144 eigenvector registers). The PSD test stays on the full
+// 12x12 matrix, as the reference runs it.
 template <int ID>
 __host__ __device__ constexpr bool translation_free() {
   return ID == YSP_ENERGY_POINT_TRIANGLE || ID == YSP_ENERGY_EDGE_EDGE ||
@@ -162,144 +174,35 @@ __device__ __forceinline__ double basis4(int a, int k) {
                 : (a <= 2 ? c2 : -3.0 * c2);
 }
 
-__device__ __forceinline__ void project_translation_free(double (&H)[78], uint32_t method) {
-  double L[78];
-#pragma unroll
-  for (int r = 0; r < 12; ++r)
-#pragma unroll
-    for (int c = 0; c <= r; ++c) L[r * (r + 1) / 2 + c] = H[upper_index<12>(c, r)];
-  if (psd_test_packed<12>(L)) return;
-  auto h12 = [&](int r, int c) { return r <= c ? H[upper_index<12>(r, c)] : H[upper_index<12>(c, r)]; };
-  double M[45];
-#pragma unroll
-  for (int k = 0; k < 3; ++k)
-#pragma unroll
-    for (int l = k; l < 3; ++l)
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          if (k == l && j < i) continue;
-          double acc = 0.0;
-#pragma unroll
-          for (int a = 0; a < 4; ++a)
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
-              acc += basis4(a, k) * basis4(b, l) * h12(3 * a + i, 3 * b + j);
-          M[upper_index<9>(3 * k + i, 3 * l + j)] = acc;
-        }
-  clamp_spectrum_packed<9>(M, method);
-  auto p9 = [&](int r, int c) { return r <= c ? M[upper_index<9>(r, c)] : M[upper_index<9>(c, r)]; };
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = a; b < 4; ++b)
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          if (a == b && j < i) continue;
-          double acc = 0.0;
-#pragma unroll
-          for (int k = 0; k < 3; ++k)
-#pragma unroll
-            for (int l = 0; l < 3; ++l)
-              acc += basis4(a, k) * basis4(b, l) * p9(3 * k + i, 3 * l + j);
-          H[upper_index<12>(3 * a + i, 3 * b + j)] = acc;
-        }
+// Elements that the evaluation does not scatter itself are held: an indefinite Hessian for
+// the projection kernel, an element whose slots are not one W-wide slot per vertex
+// (vertices driven by affine bodies, a repeated target vertex) for the general scatter,
+// or both. Slot i of a launch's list is elem[i] (element, kHeld* flags) with the packed
+// Hessian and the gradient in data, 8 slots interleaved: component c of slot i at
+// held_at<N>(i, c). A lane per slot then reads whole 64-byte pieces (one slot after the
+// other took 137 us to project what is indefinite of 122,000 hinges, this takes 116), and a
+// wavefront per slot shares its lines with the 7 slots beside it. general lists the slots of
+// the second kind.
+constexpr uint32_t kHeldIndefinite = 1u << 31, kHeldGeneral = 1u << 30;
+constexpr uint32_t kHeldElement = kHeldGeneral - 1;
+template <int N>
+__host__ __device__ constexpr int held_doubles() {
+  return N * (N + 1) / 2 + N;
 }
-
-template <int ID>
-__device__ __forceinline__ void project_element(double (&H)[Kind<ID>::N * (Kind<ID>::N + 1) / 2],
-                                                uint32_t method) {
-  if constexpr (translation_free<ID>() && Kind<ID>::A == 4 && Kind<ID>::W == 3)
-    project_translation_free(H, method);
-  else
-    project_packed<Kind<ID>::N>(H, method);
+template <int N>
+__device__ __forceinline__ size_t held_at(uint32_t slot, int c) {
+  return static_cast<size_t>(slot / 8) * (8 * held_doubles<N>()) + 8 * c + slot % 8;
 }
-
-// ----------------------------------------------------------------- slots (any size)
-// Slot groups by |perm| in first-occurrence order (hessianKernelNoProject.pyx:93-163),
-// with every slot's size and local column offset (sum of the previous slot sizes).
-template <int KT>
-struct GSlots {
-  uint32_t idx[KT];
-  uint8_t size[KT];
-  uint8_t col[KT];
-  uint8_t xbase[KT];   // first position entry of the slot's vertex
-  uint8_t amode[KT];   // 1: affine-matrix slot of an affine vertex (x_j, coefficient r_l)
-  uint8_t aff[KT];     // 1: a slot of an affine vertex (its A or its t)
-  int8_t group_first[KT];
-  uint32_t group_mask[KT];
-  int ng;
-  bool ok;
+struct Held {
+  uint32_t* counts;              // [2]: slots, general slots
+  uint32_t* elem;
+  uint32_t* general;
+  double* data;
 };
-
-template <int KT>
-__device__ __forceinline__ void load_gslots(const ScatterArgs& S, uint32_t e, int N,
-                                            GSlots<KT>& si) {
-  const uint32_t K = S.K;
-  si.ng = 0;
-  si.ok = K <= static_cast<uint32_t>(KT);
-  if (!si.ok) return;
-  int placement[KT];
-  uint32_t col = 0;
-#pragma unroll
-  for (int i = 0; i < KT; ++i) {
-    si.idx[i] = 0;
-    si.size[i] = 0;
-    si.col[i] = 0;
-    si.xbase[i] = static_cast<uint8_t>(col);
-    si.amode[i] = 0;
-    si.aff[i] = 0;
-    if (static_cast<uint32_t>(i) >= K) continue;
-    const size_t o = static_cast<size_t>(e) * K + i;
-    const uint32_t ii = S.seg_idx[o];
-    const uint32_t sz = S.seg_size[o];
-    const int pm = S.perm[o];
-    si.idx[i] = ii;
-    si.size[i] = static_cast<uint8_t>(sz);
-    si.col[i] = static_cast<uint8_t>(col);
-    col += sz;
-    if (pm == 0) continue;
-    const int p = (pm < 0 ? -pm : pm) - 1;
-    int g = -1;
-#pragma unroll
-    for (int k = 0; k < KT; ++k)
-      if (k < si.ng && placement[k] == p) g = k;
-    if (g < 0) {
-      g = si.ng++;
-#pragma unroll
-      for (int k = 0; k < KT; ++k)
-        if (k == g) {
-          placement[k] = p;
-          si.group_first[k] = static_cast<int8_t>(i);
-          si.group_mask[k] = 0;
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < KT; ++k)
-      if (k == g) si.group_mask[k] |= 1u << i;
-  }
-  if (N >= 0 && col != static_cast<uint32_t>(N)) si.ok = false;   // slots tile the DoFs
-}
 
 template <int N>
 __device__ __forceinline__ double hget(const double (&H)[N * (N + 1) / 2], int i, int j) {
   return i <= j ? H[upper_index<N>(i, j)] : H[upper_index<N>(j, i)];
-}
-
-// Position entry and coefficient of entry k of slot i (identity unless the slot is the
-// affine matrix of an affine vertex).
-template <int KT>
-__device__ __forceinline__ int xmap(const GSlots<KT>& si, const double (*r)[3], int i, int k,
-                                    double& c) {
-  if (si.amode[i]) {
-    c = r[si.xbase[i] / 3][k % 3];
-    return si.xbase[i] + k / 3;
-  }
-  c = 1.0;
-  return si.xbase[i] + k;
 }
 
 // Per-workgroup sums of the contended destinations of the general kernel (atomic mode):
@@ -358,86 +261,208 @@ __device__ __forceinline__ void hot_flush(HotTable& t, const ScatterArgs& S) {
     atomic_add_f64(S.gradient + t.gkey[j] + o, t.gval[j][o]);
   }
 }
+// The general scatter: one wavefront per held element, any slot sizes, vertices of affine
+// bodies. Slot groups by |perm| in first-occurrence order (hessianKernelNoProject.pyx:
+// 93-163); lanes hold the slots while the groups are found, then the entries of one block
+// after the other, with the element's Hessian, gradient and slots in LDS. (One lane per
+// element with run-time indices put Hessian and slots in scratch memory: 1.2 ms for 7,000
+// tets of affine bodies, 0.9 ms for 42,000 point-triangle and 0.8 ms for the edge-edge
+// pairs of the same scene; these lists now take 70 us each.)
+template <int N, int KT>
+struct ElementLds {
+  double h[N * (N + 1) / 2 + N];     // packed Hessian, then the gradient
+  double r[8][3];                    // rest positions of affine vertices
+  uint32_t idx[KT];
+  uint32_t members[KT];              // per group: its slots
+  uint32_t diag[KT];                 // per group: offset in the diagonal blocks
+  uint8_t size[KT], col[KT], xbase[KT], amode[KT], aff[KT], head[KT];
+};
 
-template <int KT, int N>
-__device__ __forceinline__ void scatter_generic(const ScatterArgs& S, uint32_t e,
-                                                const GSlots<KT>& si, const double (*r)[3],
-                                                const double (&g)[N],
-                                                const double (&H)[N * (N + 1) / 2],
-                                                HotTable* ht) {
-  // gradient
-  if (S.grad_staging) {
-    double* out = S.grad_staging + static_cast<size_t>(e) * S.grad_local;
+// LDS written by some lanes of a wavefront and then read by others of the same wavefront.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Position entry and coefficient of entry k of slot i (identity unless the slot is the
+// affine matrix of an affine vertex).
+template <typename L>
+__device__ __forceinline__ int xmap(const L& el, int i, int k, double& c) {
+  if (el.amode[i]) {
+    c = el.r[el.xbase[i] / 3][k % 3];
+    return el.xbase[i] + k / 3;
+  }
+  c = 1.0;
+  return el.xbase[i] + k;
+}
+
+constexpr unsigned kGB = 256;
+template <int A, int W, int KT>
+__global__ void __launch_bounds__(kGB)
+    energy_scatter_kernel(UnionView P, AffineView AF, const uint32_t* __restrict__ e2v,
+                          ScatterArgs S, int* __restrict__ flags, Held held) {
+  constexpr int N = A * W, NH = N * (N + 1) / 2;
+  static_assert(KT <= 64 && A <= 8, "slots and vertices of an element");
+  __shared__ HotTable table;
+  __shared__ ElementLds<N, KT> els[kGB / 64];
+  const bool hot = AF.mask && !S.block_staging;    // uniform over the grid
+  if (hot) hot_init(table);
+  ElementLds<N, KT>& el = els[threadIdx.x / 64];
+  const int lane = threadIdx.x % 64;
+  const uint32_t count = held.counts[1];
+  const uint32_t per = (count + gridDim.x - 1) / gridDim.x;   // a workgroup's run of the list
+  const uint32_t end = min(count, (blockIdx.x + 1) * per);
+  for (uint32_t i0 = blockIdx.x * per + threadIdx.x / 64; i0 < end; i0 += kGB / 64) {
+    const uint32_t slot = held.general[i0];
+    const uint32_t e = held.elem[slot] & kHeldElement;
+    const int K = static_cast<int>(S.K);
+    bool ok = K <= KT && !(S.block_staging && (W != 3 || AF.mask));
+    // lane i: slot i
+    uint32_t ii = 0, sz = 0;
+    int place = -1;
+    if (ok && lane < K) {
+      const size_t o = static_cast<size_t>(e) * S.K + lane;
+      ii = S.seg_idx[o];
+      sz = S.seg_size[o];
+      const int pm = S.perm[o];
+      place = pm == 0 ? -1 : (pm < 0 ? -pm : pm) - 1;
+    }
+    for (int i = lane; i < held_doubles<N>(); i += 64) el.h[i] = held.data[held_at<N>(slot, i)];
+    uint32_t col = 0, total = 0, members = 0;
 #pragma unroll
-    for (int i = 0; i < KT; ++i)
-      for (int k = 0; k < si.size[i]; ++k) {
-        double c;
-        const int x = xmap(si, r, i, k, c);
-        out[si.col[i] + k] = c * g[x];
+    for (int j = 0; j < KT; ++j) {
+      const uint32_t sj = __shfl(sz, j);
+      const int pj = __shfl(place, j);
+      if (j < lane) col += sj;
+      total += sj;
+      if (pj >= 0 && pj == place) members |= 1u << j;
+    }
+    const bool leads = members && __ffs(members) - 1 == lane;
+    const uint64_t heads = __ballot(leads);
+    const int ng = __popcll(heads);
+    uint32_t xbase = col;
+    bool amode = false, aff = false;
+    if (AF.mask) {
+      // slots of vertex a: [a Kv, (a + 1) Kv); an affine vertex owns A then t
+      const int Kv = K / A;
+      if (Kv * A != K || W != 3) ok = false;
+      if (ok && lane < K) {
+        const int a = lane / Kv, q = lane % Kv;
+        uint32_t local;
+        const uint32_t c = union_child(P, e2v[static_cast<size_t>(e) * A + a], local);
+        aff = (AF.mask >> c) & 1u;
+        xbase = 3 * a;
+        amode = aff && q == 0;
+        if (q == 0)
+          for (int k = 0; k < 3; ++k)
+            el.r[a][k] = aff ? AF.rest[c][3 * static_cast<size_t>(local) + k] : 0.0;
+        const int want = aff ? (q == 0 ? 9 : (q == 1 ? 3 : -1)) : (q == 0 ? 3 : -1);
+        if (want > 0 && sz != static_cast<uint32_t>(want)) ok = false;
+        if (want < 0 && ii >= 2) ok = false;
       }
-  } else {
-#pragma unroll
-    for (int i = 0; i < KT; ++i) {
-      if (si.idx[i] < 2) continue;
-      const uint32_t p = si.idx[i] - 2;
+    } else if (total != static_cast<uint32_t>(N)) {
+      ok = false;                                  // slots tile the DoFs
+    }
+    if (__any(!ok)) {
+      if (lane == 0) atomicOr(flags, 1);
+      continue;
+    }
+    if (lane < KT) {
+      el.idx[lane] = ii;
+      el.size[lane] = static_cast<uint8_t>(sz);
+      el.col[lane] = static_cast<uint8_t>(col);
+      el.xbase[lane] = static_cast<uint8_t>(xbase);
+      el.amode[lane] = amode;
+      el.aff[lane] = aff;
+    }
+    if (leads) {
+      const int g = lanes_below(heads);
+      el.head[g] = static_cast<uint8_t>(lane);
+      el.members[g] = members;
+      if (ii >= 2 && S.diag_blocks && !S.block_staging) el.diag[g] = diag_offset(S, ii - 2, sz);
+    }
+    // destinations of the block pairs, in coordinate order (at most 64 of them here)
+    const uint32_t cstart = S.coord_outer[e];
+    const int nt = __popcll(__ballot(leads && ii >= 2));
+    const uint32_t pairs = nt * (nt + 1) / 2;
+    uint32_t dest = 0;
+    if (!S.block_staging && static_cast<uint32_t>(lane) < pairs) dest = S.lookups[cstart + lane];
+    wave_lds_fence();
+    // gradient
+    for (int i = 0; i < K; ++i) {
+      const int n = el.size[i];
+      const uint32_t t = el.idx[i];
+      if (S.grad_staging) {
+        if (lane < n) {
+          double c;
+          const int x = xmap(el, i, lane, c);
+          S.grad_staging[static_cast<size_t>(e) * S.grad_local + el.col[i] + lane] = c * el.h[NH + x];
+        }
+        continue;
+      }
+      if (t < 2) continue;
       int gs = -1;
-      if (ht && si.aff[i] && si.size[i] <= kHotGradMax) {
-        gs = hot_slot(ht->gkey, kHotGrad, p);
-        if (gs >= 0) ht->gsize[gs] = si.size[i];
+      if (hot && el.aff[i] && n <= kHotGradMax) {
+        if (lane == 0) {
+          gs = hot_slot(table.gkey, kHotGrad, t - 2);
+          if (gs >= 0) table.gsize[gs] = n;
+        }
+        gs = __shfl(gs, 0);
       }
-      for (int k = 0; k < si.size[i]; ++k) {
+      if (lane < n) {
         double c;
-        const int x = xmap(si, r, i, k, c);
-        if (gs >= 0) atomicAdd(&ht->gval[gs][k], c * g[x]);
-        else atomic_add_f64(S.gradient + p + k, c * g[x]);
+        const int x = xmap(el, i, lane, c);
+        const double v = c * el.h[NH + x];
+        if (gs >= 0) atomicAdd(&table.gval[gs][lane], v);
+        else atomic_add_f64(S.gradient + (t - 2) + lane, v);
       }
     }
-  }
-  // Hessian blocks of every valid group pair, in coordinate order
-  uint32_t count = 0;
-  const uint32_t cstart = S.coord_outer[e];
-#pragma unroll
-  for (int gi = 0; gi < KT; ++gi) {
-    if (gi >= si.ng) continue;
-    const int fi = si.group_first[gi];
-    const uint32_t ii = si.idx[fi];
-    if (ii < 2) continue;
-    const int h = si.size[fi];
-#pragma unroll
-    for (int gj = gi; gj < KT; ++gj) {
-      if (gj >= si.ng) continue;
-      const int fj = si.group_first[gj];
-      const uint32_t jj = si.idx[fj];
-      if (jj < 2) continue;
-      const int w = si.size[fj];
-      const uint32_t coord = cstart + count;
-      double* dst = S.block_staging ? S.block_staging + 9 * static_cast<size_t>(coord)
-                                    : S.blocks + S.lookups[coord];
-      double* dd = nullptr;
-      if (!S.block_staging && gi == gj && S.diag_blocks) dd = S.diag_blocks + diag_offset(S, ii - 2, h);
-      int hs = -1;
-      if (ht && !S.block_staging && si.aff[fi] && si.aff[fj] && h * w <= kHotBlockMax) {
-        hs = hot_slot(ht->bkey, kHotBlocks, S.lookups[coord]);
-        if (hs >= 0) {
-          ht->bsize[hs] = h * w;
-          ht->bdiag[hs] = dd ? static_cast<uint32_t>(dd - S.diag_blocks) : kHotEmpty;
+    // Hessian blocks of every valid group pair, in coordinate order
+    uint32_t at = 0;
+    for (int gi = 0; gi < ng; ++gi) {
+      const int fi = el.head[gi];
+      const uint32_t ti = el.idx[fi];
+      if (ti < 2) continue;
+      const int h = el.size[fi];
+      for (int gj = gi; gj < ng; ++gj) {
+        const int fj = el.head[gj];
+        const uint32_t tj = el.idx[fj];
+        if (tj < 2) continue;
+        const int w = el.size[fj];
+        const uint32_t coord = cstart + at;
+        const uint32_t off = at < 64 ? __shfl(dest, static_cast<int>(at))
+                                     : (S.block_staging ? 0u : S.lookups[coord]);
+        ++at;
+        double* dst = S.block_staging ? S.block_staging + 9 * static_cast<size_t>(coord) : S.blocks + off;
+        double* dd = !S.block_staging && gi == gj && S.diag_blocks ? S.diag_blocks + el.diag[gi] : nullptr;
+        int hs = -1;
+        if (hot && el.aff[fi] && el.aff[fj] && h * w <= kHotBlockMax) {
+          if (lane == 0) {
+            hs = hot_slot(table.bkey, kHotBlocks, off);
+            if (hs >= 0) {
+              table.bsize[hs] = h * w;
+              table.bdiag[hs] = dd ? el.diag[gi] : kHotEmpty;
+            }
+          }
+          hs = __shfl(hs, 0);
         }
-      }
-      const bool tr = !(ii < jj);
-      for (int k = 0; k < h; ++k)
-        for (int l = 0; l < w; ++l) {
+        const bool tr = !(ti < tj);
+        const uint32_t inv = 65536u / w + 1;       // t / w for t < 144, w <= 12
+        for (int t = lane; t < h * w; t += 64) {
+          const int k = static_cast<int>((t * inv) >> 16), l = t - k * w;
           double v = 0.0;
-#pragma unroll
-          for (int a = 0; a < KT; ++a) {
-            if (!((si.group_mask[gi] >> a) & 1u) || si.size[a] == 0) continue;
+          for (uint32_t ma = el.members[gi]; ma; ma &= ma - 1) {
+            const int a = __ffs(ma) - 1;
+            if (el.size[a] == 0) continue;
             double ca;
-            const int xa = xmap(si, r, a, k, ca);
-#pragma unroll
-            for (int b = 0; b < KT; ++b) {
-              if (!((si.group_mask[gj] >> b) & 1u) || si.size[b] == 0) continue;
+            const int xa = xmap(el, a, k, ca);
+            for (uint32_t mb = el.members[gj]; mb; mb &= mb - 1) {
+              const int b = __ffs(mb) - 1;
+              if (el.size[b] == 0) continue;
               double cb;
-              const int xb = xmap(si, r, b, l, cb);
-              v += ca * cb * hget<N>(H, xa, xb);
+              const int xb = xmap(el, b, l, cb);
+              const int lo = min(xa, xb), hi = max(xa, xb);
+              v += ca * cb * el.h[upper_index<N>(lo, hi)];
             }
           }
           // stored block: rows of the lower global index; (l, k) of a transposed block
@@ -445,15 +470,17 @@ __device__ __forceinline__ void scatter_generic(const ScatterArgs& S, uint32_t e
           if (S.block_staging) {
             dst[o] = v;
           } else if (hs >= 0) {
-            atomicAdd(&ht->bval[hs][o], v);
+            atomicAdd(&table.bval[hs][o], v);
           } else {
             atomic_add_f64(dst + o, v);
             if (dd) atomic_add_f64(dd + o, v);
           }
         }
-      ++count;
+      }
     }
+    wave_lds_fence();                              // before the next element overwrites el
   }
+  if (hot) hot_flush(table, S);
 }
 
 template <int ID>
@@ -479,7 +506,8 @@ __device__ __forceinline__ void scene_params(const double* sp, const double* x, 
   if constexpr (ID == YSP_ENERGY_BARAFF_WITKIN) bw_stretch_coefficients(x, p, s[3], s[4]);
 }
 
-// Energy, gradient and (projected) packed Hessian of one element.
+// Energy, gradient and packed Hessian of one element (not projected, but for the quadratic
+// form, whose projection acts on its inner Hessian).
 template <int ID>
 __device__ __forceinline__ void element_eval(const double (&x)[Kind<ID>::N], const double* p,
                                              const double* sp, uint32_t method, double& E,
@@ -491,83 +519,7 @@ __device__ __forceinline__ void element_eval(const double (&x)[Kind<ID>::N], con
     double s[Kind<ID>::S];
     scene_params<ID>(sp, x, p, s);
     Kind<ID>::eval(x, p, s, E, g, H);
-    if (method != 0) project_element<ID>(H, method);
   }
-}
-
-// One element through the general slot bookkeeping (any slot sizes, affine vertices).
-template <int ID, int KT>
-__device__ __forceinline__ void eval_element_general(const UnionView& P, const AffineView& AF,
-                                                     const uint32_t* __restrict__ e2v, uint32_t e,
-                                                     const double* __restrict__ ep,
-                                                     const double* __restrict__ sp, uint32_t method,
-                                                     const ScatterArgs& SA,
-                                                     int* __restrict__ error_flag,
-                                                     HotTable* ht) {
-  using T = Kind<ID>;
-  GSlots<KT> si;
-  load_gslots<KT>(SA, e, AF.mask ? -1 : T::N, si);
-  double r[T::A][3];
-  if (AF.mask) {
-    // slots of vertex a: [a Kv, (a + 1) Kv); an affine vertex owns A then t
-    const int Kv = static_cast<int>(SA.K) / T::A;
-    if (Kv * T::A != static_cast<int>(SA.K) || T::W != 3) si.ok = false;
-#pragma unroll
-    for (int a = 0; a < T::A; ++a) {
-      uint32_t local;
-      const uint32_t c = union_child(P, e2v[static_cast<size_t>(e) * T::A + a], local);
-      const bool aff = (AF.mask >> c) & 1u;
-      r[a][0] = r[a][1] = r[a][2] = 0.0;
-      if (aff) {
-        const double* rr = AF.rest[c] + 3 * static_cast<size_t>(local);
-        r[a][0] = rr[0];
-        r[a][1] = rr[1];
-        r[a][2] = rr[2];
-      }
-#pragma unroll
-      for (int q = 0; q < KT; ++q) {
-        if (q >= Kv) continue;
-        const int i = a * Kv + q;
-        if (i >= KT) continue;
-        si.xbase[i] = static_cast<uint8_t>(3 * a);
-        si.amode[i] = aff && q == 0;
-        si.aff[i] = aff;
-        const int want = aff ? (q == 0 ? 9 : (q == 1 ? 3 : -1)) : (q == 0 ? 3 : -1);
-        if (want > 0 && si.size[i] != want) si.ok = false;
-        if (want < 0 && si.idx[i] >= 2) si.ok = false;
-      }
-    }
-  }
-  if (!si.ok || (SA.block_staging && (T::W != 3 || AF.mask))) {
-    atomicOr(error_flag, 1);
-    return;
-  }
-  double x[T::N];
-  gather<ID>(P, e2v, e, x);
-  const double* p = ep + static_cast<size_t>(e) * T::P;
-  double E, g[T::N], H[T::N * (T::N + 1) / 2];
-  element_eval<ID>(x, p, sp, method, E, g, H);
-  scatter_generic<KT, T::N>(SA, e, si, r, g, H, ht);
-}
-
-// General kernel: every element (queue == nullptr) or the elements queued by the vertex
-// kernel (count in flags[1]), in a grid-stride loop. With affine children and atomic
-// assembly, the affine destinations of the workgroup's elements are summed in LDS first.
-constexpr unsigned kGB = 256;
-template <int ID, int KT>
-__global__ void __launch_bounds__(kGB)
-    energy_eval_kernel(UnionView P, AffineView AF, const uint32_t* __restrict__ e2v, uint32_t n,
-                       const double* __restrict__ ep, const double* __restrict__ sp,
-                       uint32_t method, ScatterArgs SA, int* __restrict__ flags,
-                       const uint32_t* __restrict__ queue) {
-  __shared__ HotTable table;
-  const bool hot = AF.mask && !SA.block_staging;   // uniform over the grid
-  if (hot) hot_init(table);
-  const uint32_t count = queue ? static_cast<uint32_t>(flags[1]) : n;
-  for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < count; t += gridDim.x * blockDim.x)
-    eval_element_general<ID, KT>(P, AF, e2v, queue ? queue[t] : t, ep, sp, method, SA, flags,
-                                 hot ? &table : nullptr);
-  if (hot) hot_flush(table, SA);
 }
 
 // ----------------------------------------------------------------- vertex fast path
@@ -658,13 +610,13 @@ __device__ __forceinline__ void load_vslots(const ScatterArgs& S, uint32_t e, VS
   }
 }
 
-// Gradient segments and Hessian blocks of a vertex-layout element (the semantics of
-// scatter_generic: pair of target-group ranks lo <= hi at coordinate coordStart +
+// Gradient segments and Hessian blocks of a vertex-layout element (the semantics of the
+// general scatter: pair of target-group ranks lo <= hi at coordinate coordStart +
 // lo*n - lo(lo-1)/2 + (hi-lo), block oriented with the rows of the smaller target index).
 template <int NV, int W, int N>
-__device__ __forceinline__ void scatter_vertex(const ScatterArgs& S, uint32_t e,
-                                               const VSlots<NV>& vs, const double (&g)[N],
-                                               const double (&H)[N * (N + 1) / 2]) {
+__device__ __forceinline__ void scatter_vertex_gradient(const ScatterArgs& S, uint32_t e,
+                                                        const VSlots<NV>& vs,
+                                                        const double (&g)[N]) {
 #pragma unroll
   for (int a = 0; a < NV; ++a) {
     if (S.grad_staging ? !vs.has[a] : (!vs.has[a] || vs.idx[a] < 2)) continue;
@@ -678,6 +630,12 @@ __device__ __forceinline__ void scatter_vertex(const ScatterArgs& S, uint32_t e,
       for (int k = 0; k < W; ++k) atomic_add_f64(S.gradient + p + k, g[W * a + k]);
     }
   }
+}
+
+// block(a, b, B): the W x W block of local vertices a <= b.
+template <int NV, int W, typename BlockFn>
+__device__ __forceinline__ void scatter_vertex_blocks(const ScatterArgs& S, uint32_t e,
+                                                      const VSlots<NV>& vs, BlockFn block) {
   const uint32_t cstart = S.coord_outer[e];
   const int n = vs.ntarget;
 #pragma unroll
@@ -685,6 +643,8 @@ __device__ __forceinline__ void scatter_vertex(const ScatterArgs& S, uint32_t e,
 #pragma unroll
     for (int b = a; b < NV; ++b) {
       if (!vs.target[a] || !vs.target[b]) continue;
+      double B[W][W];
+      block(a, b, B);
       const int lo = min(vs.rank[a], vs.rank[b]), hi = max(vs.rank[a], vs.rank[b]);
       const uint32_t coord = cstart + static_cast<uint32_t>(lo * n - lo * (lo - 1) / 2 + (hi - lo));
       const bool tr = !(vs.idx[a] < vs.idx[b]);   // includes the diagonal block a == b
@@ -694,7 +654,7 @@ __device__ __forceinline__ void scatter_vertex(const ScatterArgs& S, uint32_t e,
         for (int k = 0; k < W; ++k)
 #pragma unroll
           for (int l = 0; l < W; ++l)
-            dst[tr ? l * W + k : k * W + l] = hget<N>(H, W * a + k, W * b + l);
+            dst[tr ? l * W + k : k * W + l] = B[k][l];
       } else {
         double* dst = S.blocks + S.lookups[coord];
         double* dd = nullptr;
@@ -703,7 +663,7 @@ __device__ __forceinline__ void scatter_vertex(const ScatterArgs& S, uint32_t e,
         for (int k = 0; k < W; ++k)
 #pragma unroll
           for (int l = 0; l < W; ++l) {
-            const double v = hget<N>(H, W * a + k, W * b + l);
+            const double v = B[k][l];
             const int o = tr ? l * W + k : k * W + l;
             atomic_add_f64(dst + o, v);
             if (dd) atomic_add_f64(dd + o, v);
@@ -712,22 +672,21 @@ __device__ __forceinline__ void scatter_vertex(const ScatterArgs& S, uint32_t e,
     }
 }
 
+// Evaluation of elements [first, last): gradient and Hessian, PSD test, scatter of what
+// needs nothing else. The projection lives in a kernel of its own (below): with the
+// eigensolver inlined behind the generated code every kind's kernel held both register
+// sets and two copies of the scatter.
 template <int ID, int KT>
 __global__ void __launch_bounds__(kEB)
-    energy_eval_vertex_kernel(UnionView P, const uint32_t* __restrict__ e2v, uint32_t n,
-                              const double* __restrict__ ep, const double* __restrict__ sp,
-                              uint32_t method, ScatterArgs SA, int* __restrict__ flags,
-                              uint32_t* __restrict__ queue) {
+    energy_eval_kernel(UnionView P, const uint32_t* __restrict__ e2v, uint32_t first, uint32_t last,
+                       const double* __restrict__ ep, const double* __restrict__ sp,
+                       uint32_t method, ScatterArgs SA, int* __restrict__ flags, Held held) {
   using T = Kind<ID>;
-  const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
+  const uint32_t e = first + blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= last) return;
   VSlots<T::A> vs;
   load_vslots<KT, T::A, T::W>(SA, e, vs);
-  if (!vs.ok) {
-    queue[wave_reserve(reinterpret_cast<uint32_t*>(flags) + 1, 1u)] = e;
-    return;
-  }
-  if (SA.block_staging && T::W != 3) {
+  if (vs.ok && SA.block_staging && T::W != 3) {
     atomicOr(flags, 1);
     return;
   }
@@ -736,7 +695,117 @@ __global__ void __launch_bounds__(kEB)
   const double* p = ep + static_cast<size_t>(e) * T::P;
   double E, g[T::N], H[T::N * (T::N + 1) / 2];
   element_eval<ID>(x, p, sp, method, E, g, H);
-  scatter_vertex<T::A, T::W, T::N>(SA, e, vs, g, H);
+  bool psd = true;
+  if constexpr (ID != YSP_ENERGY_QUADRATIC_FORM)
+    if (method != 0) psd = is_psd<T::N>(H);
+  if (vs.ok) {
+    scatter_vertex_gradient<T::A, T::W, T::N>(SA, e, vs, g);
+    if (psd) {
+      scatter_vertex_blocks<T::A, T::W>(SA, e, vs, [&](int a, int b, double (&B)[T::W][T::W]) {
+#pragma unroll
+        for (int k = 0; k < T::W; ++k)
+#pragma unroll
+          for (int l = 0; l < T::W; ++l) B[k][l] = hget<T::N>(H, T::W * a + k, T::W * b + l);
+      });
+      return;
+    }
+  }
+  const uint32_t slot = wave_reserve(held.counts, 1u);
+  held.elem[slot] = e | (psd ? 0u : kHeldIndefinite) | (vs.ok ? 0u : kHeldGeneral);
+#pragma unroll
+  for (int i = 0; i < T::N * (T::N + 1) / 2; ++i) held.data[held_at<T::N>(slot, i)] = H[i];
+  if (!vs.ok) {
+    held.general[wave_reserve(held.counts + 1, 1u)] = slot;
+#pragma unroll
+    for (int i = 0; i < T::N; ++i)
+      held.data[held_at<T::N>(slot, T::N * (T::N + 1) / 2 + i)] = g[i];
+  }
+}
+
+// Projection of the held indefinite Hessians: scattered (vertex layouts) or written back
+// for the general scatter. kFree: in the translation-free complement of four vertices.
+template <int A, int W, int KT, bool kFree>
+__global__ void __launch_bounds__(kEB)
+    energy_project_kernel(uint32_t method, ScatterArgs SA, Held held) {
+  constexpr int N = A * W, P = N * (N + 1) / 2;
+  const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
+  if (slot >= held.counts[0]) return;
+  const uint32_t word = held.elem[slot];
+  if (!(word & kHeldIndefinite)) return;
+  constexpr int R = kFree ? 9 : N;               // dimension of the eigenproblem
+  double D[R * (R + 1) / 2];                     // then the change of its spectrum
+  if constexpr (kFree) {
+    static_assert(A == 4 && W == 3, "four vertices");
+    double H[P];
+#pragma unroll
+    for (int i = 0; i < P; ++i) H[i] = held.data[held_at<N>(slot, i)];
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int l = k; l < 3; ++l)
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            if (k == l && j < i) continue;
+            double acc = 0.0;
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+#pragma unroll
+              for (int b = 0; b < 4; ++b)
+                acc += basis4(a, k) * basis4(b, l) * hget<12>(H, 3 * a + i, 3 * b + j);
+            D[upper_index<9>(3 * k + i, 3 * l + j)] = acc;
+          }
+  } else {
+#pragma unroll
+    for (int i = 0; i < P; ++i) D[i] = held.data[held_at<N>(slot, i)];
+  }
+  clamp_change_packed<R>(D, method);
+  // the Hessian again: not kept in registers across the eigensolver (the compiler must not
+  // know that it is the same slot)
+  uint32_t again = slot;
+  asm volatile("" : "+v"(again));
+  double* data = held.data + held_at<N>(again, 0);
+  auto block = [&](int a, int b, double (&B)[W][W]) {
+#pragma unroll
+    for (int i = 0; i < W; ++i)
+#pragma unroll
+      for (int j = 0; j < W; ++j) {
+        const int r = W * a + i, c = W * b + j;
+        double v = data[8 * (r <= c ? upper_index<N>(r, c) : upper_index<N>(c, r))];
+        if constexpr (kFree) {
+#pragma unroll
+          for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int l = 0; l < 3; ++l) {
+              const double w = basis4(a, k) * basis4(b, l);
+              if (w != 0.0) v = fma(w, hget<9>(D, 3 * k + i, 3 * l + j), v);
+            }
+        } else {
+          v += hget<R>(D, r, c);
+        }
+        B[i][j] = v;
+      }
+  };
+  if (word & kHeldGeneral) {
+#pragma unroll
+    for (int a = 0; a < A; ++a)
+#pragma unroll
+      for (int b = a; b < A; ++b) {
+        double B[W][W];
+        block(a, b, B);
+#pragma unroll
+        for (int i = 0; i < W; ++i)
+#pragma unroll
+          for (int j = 0; j < W; ++j)
+            if (a < b || j >= i) data[8 * upper_index<N>(W * a + i, W * b + j)] = B[i][j];
+      }
+    return;
+  }
+  const uint32_t e = word & kHeldElement;
+  VSlots<A> vs;
+  load_vslots<KT, A, W>(SA, e, vs);
+  scatter_vertex_blocks<A, W>(SA, e, vs, block);
 }
 
 template <int ID>
@@ -755,22 +824,33 @@ __global__ void __launch_bounds__(kEB)
   energy[e] = E;
 }
 
+// Elements per round of evaluation, projection and general scatter: what a round holds (at
+// most 94 MB) stays in the Infinity Cache between its kernels.
+constexpr uint32_t kHeldRound = 131072;
+
 template <int ID>
 int launch_eval(const UnionView& U, const AffineView& AF, const uint32_t* e2v, uint32_t n,
                 const double* ep, const double* sp, uint32_t method, const ScatterArgs& SA,
-                int* flags, uint32_t* queue, hipStream_t s) {
-  const dim3 g(grid_for(n, kEB)), b(kEB);
+                int* flags, uint32_t* elem, uint32_t* general, double* data, hipStream_t s) {
+  using T = Kind<ID>;
   auto run = [&](auto kt) {
     constexpr int KT = decltype(kt)::value;
-    // vertex-layout elements in the fast kernel; the others (affine-driven vertices, other
-    // slot layouts) are queued for the general kernel: a small grid-stride launch when
-    // the queue is usually empty, a full grid when the union has affine children
-    hipLaunchKernelGGL((energy_eval_vertex_kernel<ID, KT>), g, b, 0, s, U, e2v, n, ep, sp, method,
-                       SA, flags, queue);
-    const unsigned gg = grid_for(n, kGB);
-    const unsigned qg = AF.mask ? gg : std::min<unsigned>(gg, 64);
-    hipLaunchKernelGGL((energy_eval_kernel<ID, KT>), dim3(qg), dim3(kGB), 0, s, U, AF, e2v, n, ep,
-                       sp, method, SA, flags, queue);
+    for (uint32_t first = 0, round = 0; first < n; first += kHeldRound, ++round) {
+      const uint32_t m = std::min(kHeldRound, n - first);
+      const Held held{reinterpret_cast<uint32_t*>(flags) + 1 + 2 * round, elem, general, data};
+      const dim3 g(grid_for(m, kEB)), b(kEB);
+      hipLaunchKernelGGL((energy_eval_kernel<ID, KT>), g, b, 0, s, U, e2v, first, first + m, ep, sp,
+                         method, SA, flags, held);
+      if (method != 0 && ID != YSP_ENERGY_QUADRATIC_FORM)
+        hipLaunchKernelGGL((energy_project_kernel<T::A, T::W, KT, (translation_free<ID>() && T::A == 4 &&
+                                                                   T::W == 3)>),
+                           g, b, 0, s, method, SA, held);
+      // usually nothing to do, or everything that an affine body drives
+      const unsigned want = grid_for(m, kGB / 64);
+      hipLaunchKernelGGL((energy_scatter_kernel<T::A, T::W, KT>),
+                         dim3(std::min<unsigned>(want, AF.mask ? 1024 : 64)), dim3(kGB), 0, s, U, AF,
+                         e2v, SA, flags, held);
+    }
   };
   if (SA.K <= 8) run(std::integral_constant<int, 8>());
   else run(std::integral_constant<int, kSlotsMax>());
@@ -808,10 +888,17 @@ int eval_energy(const ysp_union_f64* positions, const ysp_affine_children* affin
   if (n == 0) return YSP_OK;
   if (int rc = check_view(positions, Kind<ID>::W, who)) return rc;
   hipStream_t s = as_stream(stream);
-  int* flag = static_cast<int*>(scratch(34, 2 * sizeof(int)));
-  uint32_t* queue = static_cast<uint32_t*>(scratch(46, sizeof(uint32_t) * n));
-  if (!flag || !queue) return YSP_ERR_HIP;
-  YSP_CHECK(hipMemsetAsync(flag, 0, 2 * sizeof(int), s));
+  if (n > kHeldElement) {
+    ysp_set_error(__FILE__, __LINE__, who);
+    return YSP_ERR_ARG;
+  }
+  const uint32_t rounds = (n + kHeldRound - 1) / kHeldRound, most = std::min(n, kHeldRound);
+  int* flag = static_cast<int*>(scratch(34, (1 + 2 * rounds) * sizeof(int)));
+  uint32_t* elem = static_cast<uint32_t*>(scratch(46, 2 * sizeof(uint32_t) * most));
+  double* data = static_cast<double*>(
+      scratch(130, sizeof(double) * held_doubles<Kind<ID>::N>() * (static_cast<size_t>(most) + 8)));
+  if (!flag || !elem || !data) return YSP_ERR_HIP;
+  YSP_CHECK(hipMemsetAsync(flag, 0, (1 + 2 * rounds) * sizeof(int), s));
   const UnionView U = make_view(positions);
   const ScatterArgs SA = make_scatter(out);
   AffineView AF{};
@@ -827,7 +914,7 @@ int eval_energy(const ysp_union_f64* positions, const ysp_affine_children* affin
     }
   }
   launch_eval<ID>(U, AF, elem2v, n, element_params, scene_params, projection_method, SA, flag,
-                  queue, s);
+                  elem, elem + most, data, s);
   YSP_CHECK_LAUNCH();
   return defer_flag_check(flag, s, "element energy: slot layout does not match the element's vertices");
 }
