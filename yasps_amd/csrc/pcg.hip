@@ -5,6 +5,8 @@
 //   (2) alpha = rz / pAp, x += alpha p, r -= alpha q, q = 0, z = M^-1 r and the partial
 //       dots r.z, r.r (one pass per diagonal block);
 //   (3) beta = rz_new / rz_old, p = z + beta p and the convergence test.
+// Over a full 3x3 block-CSR (ysp_pcg_solve_full) an iteration is two: (3) is part of (1),
+// which forms p = z + beta p_old where it reads it.
 // Scalars live in rotating sets (k mod 3) so that every kernel of iteration k reads
 // complete sums and no kernel overwrites a set another kernel of the same launch reads.
 // Each dot is a set of 64 partial-sum slots (one per 128-byte line, workgroup w adds into
@@ -19,6 +21,8 @@
 #include "values.hpp"
 
 #include <algorithm>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 namespace ysp {
@@ -102,33 +106,46 @@ __device__ __forceinline__ void apply_block(const double* __restrict__ minv, con
 
 constexpr int kVecBlock = 256;
 
-// One diagonal block of the update: x += alpha p, r -= alpha q, q = 0, z = Minv r, and
-// its r.z, r.r terms (same arithmetic order as apply_block).
-template <int S>
-__device__ __forceinline__ void update_block(const double* __restrict__ minv, uint32_t dof0,
-                                             double alpha, double* __restrict__ x,
-                                             double* __restrict__ r, const double* __restrict__ p,
-                                             double* __restrict__ q, double* __restrict__ z,
-                                             double& rz, double& rr) {
-  double rl[S];
+// One diagonal block of the update: x += alpha p, r -= alpha q, z = Minv r and its r.z, r.r
+// terms (same arithmetic order as apply_block); q = 0 with kClear, for products that add.
+template <int S, bool kClear>
+struct UpdateBlock {
+  double m[S * S], xl[S], rl[S], pl[S], ql[S];
+  __device__ __forceinline__ void load(const double* __restrict__ minv, uint32_t dof0,
+                                       const double* __restrict__ x, const double* __restrict__ r,
+                                       const double* __restrict__ p, const double* __restrict__ q) {
 #pragma unroll
-  for (int i = 0; i < S; ++i) {
-    const uint32_t d = dof0 + i;
-    x[d] = x[d] + p[d] * alpha;
-    rl[i] = r[d] - q[d] * alpha;
-    r[d] = rl[i];
-    q[d] = 0.0;
+    for (int i = 0; i < S; ++i) {
+      xl[i] = x[dof0 + i];
+      rl[i] = r[dof0 + i];
+      pl[i] = p[dof0 + i];
+      ql[i] = q[dof0 + i];
+    }
+#pragma unroll
+    for (int i = 0; i < S * S; ++i) m[i] = minv[i];
   }
+  __device__ __forceinline__ void step(uint32_t dof0, double alpha, double* __restrict__ x,
+                                       double* __restrict__ r, double* __restrict__ q,
+                                       double* __restrict__ z, double& rz, double& rr) {
 #pragma unroll
-  for (int i = 0; i < S; ++i) {
-    double acc = 0.0;
+    for (int i = 0; i < S; ++i) {
+      const uint32_t d = dof0 + i;
+      x[d] = xl[i] + pl[i] * alpha;
+      rl[i] = rl[i] - ql[i] * alpha;
+      r[d] = rl[i];
+      if (kClear) q[d] = 0.0;
+    }
 #pragma unroll
-    for (int j = 0; j < S; ++j) acc += minv[i * S + j] * rl[j];
-    z[dof0 + i] = acc;
-    rz += rl[i] * acc;
-    rr += rl[i] * rl[i];
+    for (int i = 0; i < S; ++i) {
+      double acc = 0.0;
+#pragma unroll
+      for (int j = 0; j < S; ++j) acc += m[i * S + j] * rl[j];
+      z[dof0 + i] = acc;
+      rz += rl[i] * acc;
+      rr += rl[i] * rl[i];
+    }
   }
-}
+};
 
 __global__ void __launch_bounds__(kVecBlock)
     init_kernel(DiagLayout L, const double* __restrict__ minv, const double* __restrict__ b,
@@ -206,18 +223,26 @@ __global__ void __launch_bounds__(256) init_finish_kernel(double* st, double tol
   }
 }
 
+// The status, the sums and the operands of the common 3-DoF blocks are asked for together:
+// one round trip to memory where three followed each other (5.7 -> 4.7 us at 11,000
+// blocks). Every wavefront forms the sums itself: no barrier before the operands' use.
+template <bool kClear>
 __global__ void __launch_bounds__(kVecBlock)
     update_kernel(DiagLayout L, const double* __restrict__ minv, double* __restrict__ x,
                   double* __restrict__ r, const double* __restrict__ p, double* __restrict__ q,
                   double* __restrict__ z, double* __restrict__ st, int k) {
-  if (st[S_STATUS] != 0.0) return;
   const int cur = k % 3, prev = (k + 2) % 3, next = (k + 1) % 3;
-  __shared__ double lds[2];
-  double v[2];
-  const int sets[2] = {SET_PAP + cur, SET_RZ + prev};
-  set_sums<2>(st, sets, lds, v);
-  const double pap = v[0], rzo = v[1];
   const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  const double status = st[S_STATUS];
+  double pap = st[set_base(SET_PAP + cur) + (threadIdx.x % 64) * kQuadSpace];
+  double rzo = st[set_base(SET_RZ + prev) + (threadIdx.x % 64) * kQuadSpace];
+  uint32_t dof0 = 0, inv0 = 0, s = 0;
+  const bool own = locate(L, t, dof0, inv0, s);
+  UpdateBlock<3, kClear> b3{};
+  if (own && s == 3) b3.load(minv + inv0, dof0, x, r, p, q);
+  if (status != 0.0) return;
+  pap = wave_sum(pap);
+  rzo = wave_sum(rzo);
   if (!isfinite(pap) || pap <= 0.0) {
     if (t == 0) {
       st[S_STATUS] = -1.0;
@@ -232,17 +257,21 @@ __global__ void __launch_bounds__(kVecBlock)
     st[set_base(SET_RR + next) + threadIdx.x * kQuadSpace] = 0.0;
   }
   double rz = 0.0, rr = 0.0;
-  uint32_t dof0, inv0, s;
-  if (locate(L, t, dof0, inv0, s)) {
+  if (own) {
+    auto block = [&](auto size) {
+      UpdateBlock<decltype(size)::value, kClear> b;
+      b.load(minv + inv0, dof0, x, r, p, q);
+      b.step(dof0, alpha, x, r, q, z, rz, rr);
+    };
     // compile-time block sizes keep the per-block arrays in registers
     switch (s) {
-      case 3: update_block<3>(minv + inv0, dof0, alpha, x, r, p, q, z, rz, rr); break;
-      case 9: update_block<9>(minv + inv0, dof0, alpha, x, r, p, q, z, rz, rr); break;
-      case 12: update_block<12>(minv + inv0, dof0, alpha, x, r, p, q, z, rz, rr); break;
-      case 1: update_block<1>(minv + inv0, dof0, alpha, x, r, p, q, z, rz, rr); break;
-      case 2: update_block<2>(minv + inv0, dof0, alpha, x, r, p, q, z, rz, rr); break;
-      case 4: update_block<4>(minv + inv0, dof0, alpha, x, r, p, q, z, rz, rr); break;
-      case 6: update_block<6>(minv + inv0, dof0, alpha, x, r, p, q, z, rz, rr); break;
+      case 3: b3.step(dof0, alpha, x, r, q, z, rz, rr); break;
+      case 9: block(std::integral_constant<int, 9>()); break;
+      case 12: block(std::integral_constant<int, 12>()); break;
+      case 1: block(std::integral_constant<int, 1>()); break;
+      case 2: block(std::integral_constant<int, 2>()); break;
+      case 4: block(std::integral_constant<int, 4>()); break;
+      case 6: block(std::integral_constant<int, 6>()); break;
       default: {
         double rl[kMaxBlock], zl[kMaxBlock];
         for (uint32_t i = 0; i < s; ++i) {
@@ -250,17 +279,29 @@ __global__ void __launch_bounds__(kVecBlock)
           x[d] = x[d] + p[d] * alpha;
           rl[i] = r[d] - q[d] * alpha;
           r[d] = rl[i];
-          q[d] = 0.0;
+          if (kClear) q[d] = 0.0;
         }
         apply_block(minv + inv0, rl, zl, s, rz, rr);
         for (uint32_t i = 0; i < s; ++i) z[dof0 + i] = zl[i];
       }
     }
   }
-  __shared__ double red[kVecBlock / 64];
-  rz = block_sum<kVecBlock>(rz, red);
-  rr = block_sum<kVecBlock>(rr, red);
+  // both partial sums in one block reduction
+  __shared__ double part[2][kVecBlock / 64];
+  rz = wave_sum(rz);
+  rr = wave_sum(rr);
+  if (threadIdx.x % 64 == 0) {
+    part[0][threadIdx.x / 64] = rz;
+    part[1][threadIdx.x / 64] = rr;
+  }
+  __syncthreads();
   if (threadIdx.x == 0) {
+    rz = rr = 0.0;
+#pragma unroll
+    for (unsigned w = 0; w < kVecBlock / 64; ++w) {
+      rz += part[0][w];
+      rr += part[1][w];
+    }
     atomic_add_f64(my_slot(st, SET_RZ + cur), rz);
     atomic_add_f64(my_slot(st, SET_RR + cur), rr);
   }
@@ -344,91 +385,162 @@ int launch_invert(const double* in, double* out, uint32_t count, uint32_t size, 
   return YSP_OK;
 }
 
-// y = A x over a mirrored full 3x3 block-CSR (component-major values, `stride` entries
-// per component): one 16-lane group per block row, every row written; with quad, the
-// workgroup's sum of x_r^T y_r goes into its partial-sum slot. `reverse` walks the rows
-// from the end: alternating directions from one product to the next, an operator larger
-// than the 256 MB Infinity Cache finds the part it streamed last still resident instead
-// of evicting it just before use (LRU over a cyclic stream never hits).
+// Products over a mirrored full 3x3 block-CSR (component-major values): one 16-lane group per
+// block row, every row written. `reverse` walks the rows from the end: alternating
+// directions from one product to the next, an operator larger than the 256 MB Infinity Cache
+// finds the part it streamed last still resident instead of evicting it just before use
+// (LRU over a cyclic stream never hits).
 constexpr unsigned kFullThreads = 256;
 constexpr unsigned kFullLanes = 16;
 constexpr unsigned kFullRows = kFullThreads / kFullLanes;
-// Rows with more entries than this (by default) go to full3_long_row_kernel (a
-// workgroup per row) so that a few long rows (the coupling rows of affine bodies) do not
+// Rows with more entries than this (by default) get a workgroup each so that a few long rows (the coupling rows of affine bodies) do not
 // set the time.
 constexpr uint32_t kLongRow = 128;
+// What kernel 1 of iteration k starts from: the sums of iteration k - 1, its convergence
+// test and beta. issue() asks for them, finish() (barrier inside, every thread of at least
+// three wavefronts) waits, so that a kernel asks for its first operands in between.
+struct DirectionState {
+  double slot, status, mode, thr, beta;
+  __device__ __forceinline__ void issue(const double* st, int k) {
+    const int prev = (k + 2) % 3, prev2 = (k + 1) % 3;
+    const int w = threadIdx.x / 64;
+    slot = 0.0;
+    if (w < 3) {
+      const int set = w == 0 ? SET_RZ + prev : (w == 1 ? SET_RZ + prev2 : SET_RR + prev);
+      slot = st[set_base(set) + (threadIdx.x % 64) * kQuadSpace];
+    }
+    status = st[S_STATUS];
+    mode = st[S_MODE];
+    thr = st[S_THR];
+  }
+  // false: the solve is over (uniform over the workgroup: one status, the same sums).
+  __device__ __forceinline__ bool finish(double* st, int k, bool lead) {
+    __shared__ double lds[4];
+    const int w = threadIdx.x / 64;
+    if (w < 3) {
+      slot = wave_sum(slot);
+      if (threadIdx.x % 64 == 0) lds[w] = slot;
+    }
+    if (threadIdx.x == 0) lds[3] = status;
+    __syncthreads();
+    const double rzn = lds[0], rzo = lds[1], rr = lds[2];
+    beta = 0.0;
+    if (lds[3] != 0.0) return false;
+    if (k == 1) return true;                       // first direction: p = z
+    if (!isfinite(rzn) || rzn < 0.0 || !isfinite(rzo) || rzo <= 0.0) {
+      if (lead) {
+        st[S_STATUS] = -1.0;
+        st[S_ITER] = k - 1;
+      }
+      return false;
+    }
+    const bool conv = (mode == 0.0 ? rzn : rr) <= thr;
+    if (lead) {
+      st[S_FINAL_RZ] = rzn;
+      st[S_FINAL_RR] = rr;
+      if (conv) {
+        st[S_STATUS] = 1.0;
+        st[S_ITER] = k - 1;
+      }
+    }
+    beta = rzn / rzo;
+    return !conv;
+  }
+};
+
+// The test alone, after the last iteration of a chunk (k: the next one).
+__global__ void __launch_bounds__(256) direction_test_kernel(double* st, int k) {
+  DirectionState D;
+  D.issue(st, k);
+  D.finish(st, k, threadIdx.x == 0);
+}
+
+// Kernel 1 of iteration k over the full block-CSR: the test of iteration k - 1, p = z +
+// beta p_old for the rows' own entries (stored to p) and, in registers, for every entry
+// gathered, q = A p and p^T q. The first num_long workgroups take a long row each, the
+// others 16 rows. The loop's kernels last a few microseconds each, as long as the gaps
+// between their launches: a direction kernel and a launch for the long rows of their own
+// made it four launches and 20.1 us of kernels per iteration at 11,000 rows, this makes it two
+// and 14.2 (direction, product and long rows 14.4 -> 9.6).
 template <typename Src>
 __global__ void __launch_bounds__(kFullThreads)
-    full3_product_kernel(const uint32_t* __restrict__ row_ptr, const uint32_t* __restrict__ col,
-                         Src vals, uint32_t nbr,
-                         uint32_t long_row, int reverse, const double* __restrict__ x,
-                         double* __restrict__ y, double* __restrict__ quad,
-                         const double* __restrict__ stop) {
-  if (stop && *stop != 0.0) return;
-  const uint32_t wg = reverse ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
-  const uint32_t r = wg * kFullRows + threadIdx.x / kFullLanes;
-  const int l = threadIdx.x % kFullLanes;
-  double y0 = 0.0, y1 = 0.0, y2 = 0.0, xq = 0.0;
-  if (r < nbr && row_ptr[r + 1] - row_ptr[r] <= long_row) {
-    const uint32_t k0 = row_ptr[r], k1 = row_ptr[r + 1];
-    for (uint32_t k = k0 + l; k < k1; k += kFullLanes) {
-      const uint32_t c = 3 * col[k];
-      const double x0 = x[c], x1 = x[c + 1], x2 = x[c + 2];
-      double b[9];
-      vals.load(k, b);
-      block_fma(b, x0, x1, x2, y0, y1, y2);
+    full3_direction_kernel(const uint32_t* __restrict__ row_ptr, const uint32_t* __restrict__ col,
+                           Src vals, uint32_t nbr, uint32_t long_row,
+                           const uint32_t* __restrict__ long_rows, uint32_t num_long, int reverse,
+                           const double* __restrict__ z, const double* __restrict__ p_old,
+                           double* __restrict__ p, double* __restrict__ q,
+                           double* __restrict__ st, int k) {
+  DirectionState D;
+  D.issue(st, k);
+  const bool is_long = blockIdx.x < num_long;
+  const uint32_t step = is_long ? kFullThreads : kFullLanes;
+  const uint32_t l = threadIdx.x % step;
+  uint32_t r;
+  if (is_long) {
+    r = long_rows[reverse ? num_long - 1 - blockIdx.x : blockIdx.x];
+  } else {
+    const uint32_t b = blockIdx.x - num_long, last = gridDim.x - num_long - 1;
+    r = (reverse ? last - b : b) * kFullRows + threadIdx.x / kFullLanes;
+  }
+  uint32_t k0 = 0, k1 = 0;
+  bool own = r < nbr;
+  if (own) {
+    k0 = row_ptr[r];
+    k1 = row_ptr[r + 1];
+    if (!is_long && k1 - k0 > long_row) {          // its workgroup is one of the first
+      own = false;
+      k1 = k0;
     }
+  }
+  // the first entry of each lane and the row's own part of the vectors, before the sums
+  uint32_t e = k0 + l;
+  double b[9], z0 = 0.0, z1 = 0.0, z2 = 0.0, o0 = 0.0, o1 = 0.0, o2 = 0.0, zr = 0.0, pr = 0.0;
+  auto fetch = [&]() {
+    const uint32_t c = 3 * col[e];
+    z0 = z[c];
+    z1 = z[c + 1];
+    z2 = z[c + 2];
+    o0 = p_old[c];
+    o1 = p_old[c + 1];
+    o2 = p_old[c + 2];
+    vals.load(e, b);
+  };
+  if (e < k1) fetch();
+  const bool writes = own && l < 3;
+  if (writes) {
+    zr = z[3 * r + l];
+    pr = p_old[3 * r + l];
+  }
+  if (!D.finish(st, k, blockIdx.x == 0 && threadIdx.x == 0)) return;
+  double y0 = 0.0, y1 = 0.0, y2 = 0.0;
+  while (e < k1) {
+    block_fma(b, z0 + o0 * D.beta, z1 + o1 * D.beta, z2 + o2 * D.beta, y0, y1, y2);
+    e += step;
+    if (e < k1) fetch();
+  }
+  __shared__ double red[kFullThreads / 64];
+  if (is_long) {
+    y0 = block_sum<kFullThreads>(y0, red);
+    y1 = block_sum<kFullThreads>(y1, red);
+    y2 = block_sum<kFullThreads>(y2, red);
+  } else {
 #pragma unroll
     for (int off = kFullLanes / 2; off > 0; off >>= 1) {
       y0 += __shfl_xor(y0, off, kFullLanes);
       y1 += __shfl_xor(y1, off, kFullLanes);
       y2 += __shfl_xor(y2, off, kFullLanes);
     }
-    if (l == 0) {
-      y[3 * r] = y0;
-      y[3 * r + 1] = y1;
-      y[3 * r + 2] = y2;
-      xq = x[3 * r] * y0 + x[3 * r + 1] * y1 + x[3 * r + 2] * y2;
-    }
   }
-  if (quad) {
-    __shared__ double red[kFullThreads / 64];
-    const double sum = block_sum<kFullThreads>(xq, red);
-    if (threadIdx.x == 0) atomic_add_f64(quad + (blockIdx.x % kQuadSlots) * kQuadSpace, sum);
+  double pq = 0.0;
+  if (writes) {
+    const double y = l == 0 ? y0 : (l == 1 ? y1 : y2);
+    pr = zr + pr * D.beta;
+    p[3 * r + l] = pr;
+    q[3 * r + l] = y;
+    pq = pr * y;
   }
-}
-
-// The rows longer than kLongRow (listed in long_rows): one workgroup per row.
-template <typename Src>
-__global__ void __launch_bounds__(kFullThreads)
-    full3_long_row_kernel(const uint32_t* __restrict__ row_ptr, const uint32_t* __restrict__ col,
-                          Src vals,
-                          const uint32_t* __restrict__ long_rows, int reverse,
-                          const double* __restrict__ x, double* __restrict__ y,
-                          double* __restrict__ quad, const double* __restrict__ stop) {
-  if (stop && *stop != 0.0) return;
-  const uint32_t r = long_rows[reverse ? gridDim.x - 1 - blockIdx.x : blockIdx.x];
-  const uint32_t k0 = row_ptr[r], k1 = row_ptr[r + 1];
-  double y0 = 0.0, y1 = 0.0, y2 = 0.0;
-  for (uint32_t k = k0 + threadIdx.x; k < k1; k += kFullThreads) {
-    const uint32_t c = 3 * col[k];
-    const double x0 = x[c], x1 = x[c + 1], x2 = x[c + 2];
-    double b[9];
-    vals.load(k, b);
-    block_fma(b, x0, x1, x2, y0, y1, y2);
-  }
-  __shared__ double red[kFullThreads / 64];
-  y0 = block_sum<kFullThreads>(y0, red);
-  y1 = block_sum<kFullThreads>(y1, red);
-  y2 = block_sum<kFullThreads>(y2, red);
-  if (threadIdx.x == 0) {
-    y[3 * r] = y0;
-    y[3 * r + 1] = y1;
-    y[3 * r + 2] = y2;
-    if (quad)
-      atomic_add_f64(quad + (blockIdx.x % kQuadSlots) * kQuadSpace,
-                     x[3 * r] * y0 + x[3 * r + 1] * y1 + x[3 * r + 2] * y2);
-  }
+  pq = block_sum<kFullThreads>(pq, red);
+  if (threadIdx.x == 0) atomic_add_f64(my_slot(st, SET_PAP + k % 3), pq);
 }
 
 // Pinned status mailbox shared by the solves issued from this process.
@@ -493,11 +605,12 @@ extern "C" int ysp_invert_diagonal_blocks(const double* diagonal_blocks, double*
 
 namespace ysp {
 namespace {
-// The PCG loop of ysp_pcg_solve over any operator: product(x, y, quad, stop) launches
-// y = A x (accumulate == 0: y is overwritten for every row; otherwise y is zero on entry
-// and receives sums), adding x^T A x into the partial-sum set quad when it is not null.
-template <typename Product>
-int generic_run(Product&& product, uint32_t max_iterations, double threshold,
+// The PCG loop over any operator, one of the two callables being nullptr: product(x, y, quad,
+// stop) adds A x to y, which is zero on entry, and x^T A x into the partial-sum set quad if
+// that is not null; direction(z, p_old, p, q, st, k) launches kernel 1 of the two-kernel
+// iteration, p alternating between two vectors.
+template <typename Product, typename Direction>
+int generic_run(Product&& product, Direction&& direction, uint32_t max_iterations, double threshold,
                 int32_t threshold_mode, const double* diagonal_blocks_inverse,
                 const uint32_t* diagonal_blocks_start, const uint32_t* diagonal_blocks_count,
                 const uint32_t* diagonal_blocks_size, const uint32_t* gradient_segments_start,
@@ -534,8 +647,10 @@ int generic_run(Product&& product, uint32_t max_iterations, double threshold,
   double* p = work + n;
   double* z = work + 2 * static_cast<size_t>(n);
   double* q = work + 3 * static_cast<size_t>(n);
+  [[maybe_unused]] double* p2 = work + 4 * static_cast<size_t>(n);
   double* x = solution;
   double* st = cg_scalars;
+  constexpr bool kFused = !std::is_same_v<std::decay_t<Direction>, std::nullptr_t>;
   const uint32_t nblocks = L.cum[num_attributes];
   const dim3 vgrid(grid_for(nblocks, kVecBlock)), vblock(kVecBlock);
   const dim3 dgrid(std::min<unsigned>(grid_for(n, kVecBlock), 2048u));
@@ -543,8 +658,14 @@ int generic_run(Product&& product, uint32_t max_iterations, double threshold,
   YSP_CHECK(hipMemsetAsync(st, 0, kStateDoubles * sizeof(double), s));
   const int have_guess = (!zero_initial_guess && initial_guess) ? 1 : 0;
   if (have_guess) {
-    YSP_CHECK(hipMemsetAsync(q, 0, sizeof(double) * n, s));
-    if (int rc = product(initial_guess, q, nullptr, nullptr)) return rc;
+    if constexpr (kFused) {
+      // the first direction of a system whose z is the guess: p2 = x0, q = A x0
+      if (int rc = direction(initial_guess, initial_guess, p2, q, st, 1)) return rc;
+      YSP_CHECK(hipMemsetAsync(st, 0, kStateDoubles * sizeof(double), s));
+    } else {
+      YSP_CHECK(hipMemsetAsync(q, 0, sizeof(double) * n, s));
+      if (int rc = product(initial_guess, q, nullptr, nullptr)) return rc;
+    }
   }
   hipLaunchKernelGGL(init_kernel, vgrid, vblock, 0, s, L, diagonal_blocks_inverse, rhs, x,
                      initial_guess, r, p, z, q, st, have_guess);
@@ -571,12 +692,21 @@ int generic_run(Product&& product, uint32_t max_iterations, double threshold,
     const uint32_t last = std::min<uint32_t>(max_iterations, k + chunk - 1);
     for (uint32_t it = k; it <= last; ++it) {
       const int cur = static_cast<int>(it % 3);
-      if (int rc = product(p, q, st + set_base(SET_PAP + cur), st + S_STATUS)) return rc;
-      hipLaunchKernelGGL(update_kernel, vgrid, vblock, 0, s, L, diagonal_blocks_inverse, x, r, p,
-                         q, z, st, static_cast<int>(it));
-      hipLaunchKernelGGL(direction_kernel, dgrid, vblock, 0, s, z, p, st, n,
-                         static_cast<int>(it));
+      if constexpr (kFused) {
+        if (int rc = direction(z, p, p2, q, st, static_cast<int>(it))) return rc;
+        std::swap(p, p2);
+      } else {
+        if (int rc = product(p, q, st + set_base(SET_PAP + cur), st + S_STATUS)) return rc;
+      }
+      hipLaunchKernelGGL(update_kernel<!kFused>, vgrid, vblock, 0, s, L, diagonal_blocks_inverse, x,
+                         r, p, q, z, st, static_cast<int>(it));
+      if constexpr (!kFused)
+        hipLaunchKernelGGL(direction_kernel, dgrid, vblock, 0, s, z, p, st, n,
+                           static_cast<int>(it));
     }
+    if constexpr (kFused)
+      hipLaunchKernelGGL(direction_test_kernel, dim3(1), dim3(256), 0, s, st,
+                         static_cast<int>(last + 1));
     YSP_CHECK_LAUNCH();
     if (int rc = read_status(box)) return rc;
     for (int i = 0; i < 8; ++i) h[i] = box[i];
@@ -626,7 +756,7 @@ extern "C" int ysp_pcg_solve(uint32_t max_iterations, double threshold, int32_t 
     if (int rc = launch_part_spmv(part, x, y, 0, quad, stop, s)) return rc;
     return launch_part_spmv(dynamic_part, x, y, 0, quad, stop, s);
   };
-  return generic_run(product, max_iterations, threshold, threshold_mode, diagonal_blocks_inverse,
+  return generic_run(product, nullptr, max_iterations, threshold, threshold_mode, diagonal_blocks_inverse,
                      diagonal_blocks_start, diagonal_blocks_count, diagonal_blocks_size,
                      gradient_segments_start, num_attributes, rhs, n, solution, initial_guess,
                      zero_initial_guess, work, cg_scalars, stats, s);
@@ -679,20 +809,15 @@ extern "C" int ysp_pcg_solve_full(uint32_t max_iterations, double threshold,
   int reverse = 0;                 // direction of the next product's row walk
   // value source (values.hpp): FP64 or FP32 copy (FP32 values, the mixed-precision inner
   // solve, are widened to FP64 as they are read) or the upper storage read in place
-  auto product = [&](const double* x, double* y, double* quad, const double* stop) -> int {
-    if (nbr == 0) return YSP_OK;
+  auto direction = [&](const double* z, const double* p_old, double* p, double* q, double* st,
+                       int k) -> int {
     if (int rc = with_values(values, values_f32, nnz, "ysp_pcg_solve_full: bad value source",
                              [&](auto vals) {
-                               using Src = decltype(vals);
-                               hipLaunchKernelGGL(full3_product_kernel<Src>,
-                                                  dim3(grid_for(nbr, kFullRows)),
+                               hipLaunchKernelGGL(full3_direction_kernel<decltype(vals)>,
+                                                  dim3(num_long_rows + grid_for(nbr, kFullRows)),
                                                   dim3(kFullThreads), 0, s, row_ptr, col, vals,
-                                                  nbr, long_row, reverse, x, y, quad, stop);
-                               if (num_long_rows)
-                                 hipLaunchKernelGGL(full3_long_row_kernel<Src>,
-                                                    dim3(num_long_rows), dim3(kFullThreads), 0, s,
-                                                    row_ptr, col, vals, long_rows, reverse, x, y,
-                                                    quad, stop);
+                                                  nbr, long_row, long_rows, num_long_rows, reverse,
+                                                  z, p_old, p, q, st, k);
                                return YSP_OK;
                              }))
       return rc;
@@ -700,7 +825,7 @@ extern "C" int ysp_pcg_solve_full(uint32_t max_iterations, double threshold,
     YSP_CHECK_LAUNCH();
     return YSP_OK;
   };
-  return generic_run(product, max_iterations, threshold, threshold_mode, diagonal_blocks_inverse,
+  return generic_run(nullptr, direction, max_iterations, threshold, threshold_mode, diagonal_blocks_inverse,
                      diagonal_blocks_start, diagonal_blocks_count, diagonal_blocks_size,
                      gradient_segments_start, num_attributes, rhs, n, solution, initial_guess,
                      zero_initial_guess, work, cg_scalars, stats, s);
