@@ -205,13 +205,21 @@ __device__ __forceinline__ double hget(const double (&H)[N * (N + 1) / 2], int i
   return i <= j ? H[upper_index<N>(i, j)] : H[upper_index<N>(j, i)];
 }
 
-// Per-workgroup sums of the contended destinations of the general kernel (atomic mode):
+// Per-workgroup sums of the contended destinations of the general scatter (atomic mode):
 // every element of an affine body adds into the same (A, A), (A, t), (t, t) blocks and the
 // same 12 gradient entries of that body, so a device-scope FP64 atomic per element and
 // entry serialises on a few addresses. Blocks coupling two affine groups and gradient
-// segments of affine groups are summed in LDS instead (LDS atomics, a few slots keyed by
-// the destination's offset) and leave with one global atomic per entry and workgroup; a
-// destination that finds no free slot takes the global atomic directly.
+// segments of affine groups are summed in LDS instead (a few slots keyed by the
+// destination's offset, found by all, with a sum for each wavefront) and leave with one
+// global atomic per entry and workgroup, the wavefronts' sums added in order: a list that
+// one workgroup takes gives the same bits every time. A destination that finds no free slot
+// takes the global atomic directly.
+constexpr unsigned kGB = 1024, kGW = kGB / 64;
+// Lists up to this length go to one workgroup: small scenes, whose other sums one wavefront
+// forms, are then assembled to the same bits every time (a stiff solve's iteration count
+// depends on them). Longer ones are spread over the chip: with 256 elements a workgroup
+// 7,000 tets and 42,000 pairs took 344 us each, spread 64.
+constexpr uint32_t kGRun = 256;
 constexpr uint32_t kHotEmpty = 0xffffffffu;
 constexpr int kHotBlocks = 8, kHotBlockMax = 81, kHotGrad = 4, kHotGradMax = 9;
 struct HotTable {
@@ -220,8 +228,8 @@ struct HotTable {
   uint32_t bdiag[kHotBlocks];   // offset in S.diag_blocks, kHotEmpty without one
   uint32_t gkey[kHotGrad];      // gradient offset
   uint32_t gsize[kHotGrad];
-  double bval[kHotBlocks][kHotBlockMax];
-  double gval[kHotGrad][kHotGradMax];
+  double bval[kGW][kHotBlocks][kHotBlockMax];
+  double gval[kGW][kHotGrad][kHotGradMax];
 };
 
 __device__ __forceinline__ int hot_slot(uint32_t* keys, int cap, uint32_t key) {
@@ -237,10 +245,8 @@ __device__ __forceinline__ int hot_slot(uint32_t* keys, int cap, uint32_t key) {
 }
 
 __device__ __forceinline__ void hot_init(HotTable& t) {
-  for (uint32_t i = threadIdx.x; i < kHotBlocks * kHotBlockMax; i += blockDim.x)
-    t.bval[i / kHotBlockMax][i % kHotBlockMax] = 0.0;
-  for (uint32_t i = threadIdx.x; i < kHotGrad * kHotGradMax; i += blockDim.x)
-    t.gval[i / kHotGradMax][i % kHotGradMax] = 0.0;
+  for (uint32_t i = threadIdx.x; i < kGW * kHotBlocks * kHotBlockMax; i += kGB) (&t.bval[0][0][0])[i] = 0.0;
+  for (uint32_t i = threadIdx.x; i < kGW * kHotGrad * kHotGradMax; i += kGB) (&t.gval[0][0][0])[i] = 0.0;
   if (threadIdx.x < kHotBlocks) t.bkey[threadIdx.x] = kHotEmpty;
   if (threadIdx.x < kHotGrad) t.gkey[threadIdx.x] = kHotEmpty;
   __syncthreads();
@@ -248,26 +254,30 @@ __device__ __forceinline__ void hot_init(HotTable& t) {
 
 __device__ __forceinline__ void hot_flush(HotTable& t, const ScatterArgs& S) {
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < kHotBlocks * kHotBlockMax; i += blockDim.x) {
+  for (uint32_t i = threadIdx.x; i < kHotBlocks * kHotBlockMax; i += kGB) {
     const uint32_t j = i / kHotBlockMax, o = i % kHotBlockMax;
     if (t.bkey[j] == kHotEmpty || o >= t.bsize[j]) continue;
-    const double v = t.bval[j][o];
+    double v = 0.0;
+    for (unsigned w = 0; w < kGW; ++w) v += t.bval[w][j][o];
     atomic_add_f64(S.blocks + t.bkey[j] + o, v);
     if (t.bdiag[j] != kHotEmpty) atomic_add_f64(S.diag_blocks + t.bdiag[j] + o, v);
   }
-  for (uint32_t i = threadIdx.x; i < kHotGrad * kHotGradMax; i += blockDim.x) {
+  for (uint32_t i = threadIdx.x; i < kHotGrad * kHotGradMax; i += kGB) {
     const uint32_t j = i / kHotGradMax, o = i % kHotGradMax;
     if (t.gkey[j] == kHotEmpty || o >= t.gsize[j]) continue;
-    atomic_add_f64(S.gradient + t.gkey[j] + o, t.gval[j][o]);
+    double v = 0.0;
+    for (unsigned w = 0; w < kGW; ++w) v += t.gval[w][j][o];
+    atomic_add_f64(S.gradient + t.gkey[j] + o, v);
   }
 }
+
 // The general scatter: one wavefront per held element, any slot sizes, vertices of affine
 // bodies. Slot groups by |perm| in first-occurrence order (hessianKernelNoProject.pyx:
 // 93-163); lanes hold the slots while the groups are found, then the entries of one block
 // after the other, with the element's Hessian, gradient and slots in LDS. (One lane per
 // element with run-time indices put Hessian and slots in scratch memory: 1.2 ms for 7,000
 // tets of affine bodies, 0.9 ms for 42,000 point-triangle and 0.8 ms for the edge-edge
-// pairs of the same scene; these lists now take 70 us each.)
+// pairs of the same scene; these lists now take 64 us each.)
 template <int N, int KT>
 struct ElementLds {
   double h[N * (N + 1) / 2 + N];     // packed Hessian, then the gradient
@@ -296,7 +306,6 @@ __device__ __forceinline__ int xmap(const L& el, int i, int k, double& c) {
   return el.xbase[i] + k;
 }
 
-constexpr unsigned kGB = 256;
 template <int A, int W, int KT>
 __global__ void __launch_bounds__(kGB)
     energy_scatter_kernel(UnionView P, AffineView AF, const uint32_t* __restrict__ e2v,
@@ -306,11 +315,13 @@ __global__ void __launch_bounds__(kGB)
   __shared__ HotTable table;
   __shared__ ElementLds<N, KT> els[kGB / 64];
   const bool hot = AF.mask && !S.block_staging;    // uniform over the grid
-  if (hot) hot_init(table);
   ElementLds<N, KT>& el = els[threadIdx.x / 64];
   const int lane = threadIdx.x % 64;
   const uint32_t count = held.counts[1];
-  const uint32_t per = (count + gridDim.x - 1) / gridDim.x;   // a workgroup's run of the list
+  // a workgroup's run of the list
+  const uint32_t per = count <= kGRun ? kGRun : (count + gridDim.x - 1) / gridDim.x;
+  if (blockIdx.x * per >= count) return;
+  if (hot) hot_init(table);
   const uint32_t end = min(count, (blockIdx.x + 1) * per);
   for (uint32_t i0 = blockIdx.x * per + threadIdx.x / 64; i0 < end; i0 += kGB / 64) {
     const uint32_t slot = held.general[i0];
@@ -413,7 +424,7 @@ __global__ void __launch_bounds__(kGB)
         double c;
         const int x = xmap(el, i, lane, c);
         const double v = c * el.h[NH + x];
-        if (gs >= 0) atomicAdd(&table.gval[gs][lane], v);
+        if (gs >= 0) table.gval[threadIdx.x / 64][gs][lane] += v;
         else atomic_add_f64(S.gradient + (t - 2) + lane, v);
       }
     }
@@ -470,7 +481,7 @@ __global__ void __launch_bounds__(kGB)
           if (S.block_staging) {
             dst[o] = v;
           } else if (hs >= 0) {
-            atomicAdd(&table.bval[hs][o], v);
+            table.bval[threadIdx.x / 64][hs][o] += v;
           } else {
             atomic_add_f64(dst + o, v);
             if (dd) atomic_add_f64(dd + o, v);
@@ -846,10 +857,9 @@ int launch_eval(const UnionView& U, const AffineView& AF, const uint32_t* e2v, u
                                                                    T::W == 3)>),
                            g, b, 0, s, method, SA, held);
       // usually nothing to do, or everything that an affine body drives
-      const unsigned want = grid_for(m, kGB / 64);
       hipLaunchKernelGGL((energy_scatter_kernel<T::A, T::W, KT>),
-                         dim3(std::min<unsigned>(want, AF.mask ? 1024 : 64)), dim3(kGB), 0, s, U, AF,
-                         e2v, SA, flags, held);
+                         dim3(std::min<unsigned>(grid_for(m, kGW), AF.mask ? 256 : 64)), dim3(kGB),
+                         0, s, U, AF, e2v, SA, flags, held);
     }
   };
   if (SA.K <= 8) run(std::integral_constant<int, 8>());
