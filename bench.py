@@ -507,8 +507,8 @@ def contact_leg(args):
 def large_operator_leg(args, n=64, steps=5):
     """The FP64 block-Jacobi Newton solve on a cube whose mirrored block-CSR (285 MB at
     n=64) does not stay in the 256 MB Infinity Cache, with the solve loop reading the
-    mirrored copy and reading the upper block storage through the entries' source words
-    (the automatic choice for such an operator). Same iterations; ms per solve."""
+    mirrored copy and reading the automatic choice for such an operator (the tiled
+    symmetric copy). Same iterations; ms per solve."""
     from yasps_amd import device as dev
     from yasps_amd.scenes import cube_scene, build_yasps_scene
     torch = dev.torch()
@@ -531,7 +531,8 @@ def large_operator_leg(args, n=64, steps=5):
         st = s0.minimizer.linearSolver.statistics
         out[source] = {"ms_per_solve": round(ms, 3), "solves_per_s": round(1e3 / ms, 2),
                        "pcg_iterations": int(st["iterations"]),
-                       "values_read": "upper storage" if hs.solve_values()[1] == 2 else "mirrored copy"}
+                       "values_read": ("mirrored copy", "", "upper storage", "tiled symmetric copy")[
+                           hs.pcg_values()[1]]}
     print(f"large operator n={n}: mirrored {out['mirrored']['ms_per_solve']} ms, "
           f"auto {out['auto']['ms_per_solve']} ms", file=sys.stderr, flush=True)
     return out
