@@ -728,15 +728,17 @@ __global__ void __launch_bounds__(kEB)
                        uint32_t method, ScatterArgs SA, int* __restrict__ flags, Held held) {
   using T = Kind<ID>;
   __shared__ WaveScatter<T::W> ws;
+  // staged blocks are 3 x 3: a launch of any other width is refused whole (no lane alone:
+  // the lanes that stay would read LDS words that those which left never wrote)
+  if (SA.block_staging && T::W != 3) {
+    if (threadIdx.x == 0) atomicOr(flags, 1);
+    return;
+  }
   const uint32_t i = first + blockIdx.x * blockDim.x + threadIdx.x;
   const bool live = i < last;                    // the wavefront scatters together
   const uint32_t e = live ? i : last - 1;
   VSlots<T::A> vs;
   load_vslots<KT, T::A, T::W>(SA, e, vs);
-  if (vs.ok && SA.block_staging && T::W != 3) {  // the lanes left have nothing to scatter here
-    atomicOr(flags, 1);
-    return;
-  }
   double x[T::N];
   gather<ID>(P, e2v, e, x);
   const double* p = ep + static_cast<size_t>(e) * T::P;
