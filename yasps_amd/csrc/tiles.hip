@@ -216,7 +216,7 @@ extern "C" int ysp_bsr3_tiles_layout(const uint32_t* row_ptr, const uint32_t* co
   const uint32_t tiles = (nv + kTileRows - 1) / kTileRows, slices = tiles * (kTileRows / 64);
   uint32_t* tile = work;
   uint32_t* local = work + nv;
-  uint32_t* key = static_cast<uint32_t*>(scratch(120, sizeof(uint32_t) * nv));
+  uint32_t* key = static_cast<uint32_t*>(scratch(131, sizeof(uint32_t) * nv));
   uint32_t* row = static_cast<uint32_t*>(scratch(121, sizeof(uint32_t) * nv));
   uint32_t* key2 = static_cast<uint32_t*>(scratch(122, sizeof(uint32_t) * nv));
   uint32_t* row2 = static_cast<uint32_t*>(scratch(123, sizeof(uint32_t) * nv));
