@@ -941,6 +941,8 @@ int eval_energy(const ysp_union_f64* positions, const ysp_affine_children* affin
     ysp_set_error(__FILE__, __LINE__, who);
     return YSP_ERR_ARG;
   }
+  const ElementScratchOrder order(s);
+  if (order.rc != YSP_OK) return order.rc;
   const uint32_t rounds = (n + kHeldRound - 1) / kHeldRound, most = std::min(n, kHeldRound);
   int* flag = static_cast<int*>(scratch(34, (1 + 2 * rounds) * sizeof(int)));
   uint32_t* elem = static_cast<uint32_t*>(scratch(46, 2 * sizeof(uint32_t) * most));

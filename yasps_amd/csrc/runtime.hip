@@ -133,3 +133,42 @@ extern "C" void ysp_release_scratch(void) {
     s.bytes = 0;
   }
 }
+
+namespace {
+std::mutex g_element_mutex;
+bool g_element_used = false;              // an evaluation was queued on g_element_stream
+hipStream_t g_element_stream = nullptr;
+hipEvent_t g_element_event = nullptr;
+
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(s, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
+}
+
+// Makes s wait for what the last evaluation's stream holds (event recorded now).
+int order_elements(hipStream_t s) {
+  if (g_element_used && g_element_stream == s) return YSP_OK;
+  if (capturing(s)) return YSP_OK;
+  if (g_element_used && !capturing(g_element_stream)) {
+    if (!g_element_event)
+      YSP_CHECK(hipEventCreateWithFlags(&g_element_event, hipEventDisableTiming));
+    // a stream that was destroyed meanwhile cannot be waited for by itself
+    if (hipEventRecord(g_element_event, g_element_stream) != hipSuccess ||
+        hipStreamWaitEvent(s, g_element_event, 0) != hipSuccess) {
+      (void)hipGetLastError();
+      YSP_CHECK(hipDeviceSynchronize());
+    }
+  }
+  g_element_used = true;
+  g_element_stream = s;
+  return YSP_OK;
+}
+}  // namespace
+
+namespace ysp {
+ElementScratchOrder::ElementScratchOrder(hipStream_t s) {
+  g_element_mutex.lock();
+  rc = order_elements(s);
+}
+ElementScratchOrder::~ElementScratchOrder() { g_element_mutex.unlock(); }
+}  // namespace ysp
