@@ -29,12 +29,21 @@ def _membranes(n, seed):
     return s0.minimizer.computeNumericValue()
 
 
-@pytest.mark.parametrize("sizes", [(200_000, 300), (300, 200_000), (20_000, 20_000)])
-def test_two_streams_keep_their_hessians(sizes):
+def _tets(n, seed):
+    """SNH tets and inertia of a cube (6 n^3 tets), many of the tets in the projection's queue."""
+    from yasps_amd.scenes import cube_scene, build_yasps_scene
+    s0, _ = build_yasps_scene(cube_scene(n, seed=seed))
+    return s0.minimizer.computeNumericValue()
+
+
+@pytest.mark.parametrize("scene,sizes", [(_membranes, (200_000, 300)), (_membranes, (300, 200_000)),
+                                         (_membranes, (20_000, 20_000)), (_tets, (32, 4)),
+                                         (_tets, (4, 32)), (_tets, (16, 16))])
+def test_two_streams_keep_their_hessians(scene, sizes):
     from yasps_amd import device as dev
     t = dev.torch()
-    print(f"element streams {sizes}", flush=True)
-    hs = [_membranes(n, k) for k, n in enumerate(sizes)]
+    print(f"element streams {scene.__name__} {sizes}", flush=True)
+    hs = [scene(n, k) for k, n in enumerate(sizes)]
     want = [(h.gradient.value.clone(), h.blocks_flattened.clone()) for h in hs]
     streams = [t.cuda.Stream() for _ in hs]
     t.cuda.synchronize()

@@ -37,7 +37,7 @@ int defer_flag_check(const int* flag, hipStream_t s, const char* what);
 // Each slot is an independent buffer so nested users do not alias.
 void* scratch(int slot, size_t bytes);
 
-// Element evaluations hand Hessians and counts from one launch to the next through scratch. While
+// Element evaluations hand Hessians, queues and counts from one launch to the next through scratch. While
 // one of these lives, no other evaluation is being queued (host lock), and an evaluation on
 // another stream than the last one's waits on the device for what is queued there: without it
 // the second call cleared the counts and overwrote the Hessians that the first had yet to

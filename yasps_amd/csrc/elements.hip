@@ -618,6 +618,8 @@ extern "C" int ysp_eval_snh_tet(const ysp_union_f64* positions, const uint32_t* 
     return YSP_ERR_ARG;
   }
   hipStream_t s = as_stream(stream);
+  const ElementScratchOrder order(s);
+  if (order.rc != YSP_OK) return order.rc;
   uint32_t* queue = static_cast<uint32_t*>(scratch(30, sizeof(uint32_t) * num_tets));
   uint32_t* qcount = static_cast<uint32_t*>(scratch(31, 2 * sizeof(uint32_t) + sizeof(int)));
   if (!queue || !qcount) return YSP_ERR_HIP;
@@ -697,6 +699,8 @@ extern "C" int ysp_eval_inertia(const double* position, const double* last_posit
     return YSP_ERR_ARG;
   }
   hipStream_t s = as_stream(stream);
+  const ElementScratchOrder order(s);
+  if (order.rc != YSP_OK) return order.rc;
   int* flag = static_cast<int*>(scratch(32, sizeof(int)));
   if (!flag) return YSP_ERR_HIP;
   YSP_CHECK(hipMemsetAsync(flag, 0, sizeof(int), s));
