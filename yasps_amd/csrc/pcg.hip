@@ -5,8 +5,8 @@
 //   (2) alpha = rz / pAp, x += alpha p, r -= alpha q, q = 0, z = M^-1 r and the partial
 //       dots r.z, r.r (one pass per diagonal block);
 //   (3) beta = rz_new / rz_old, p = z + beta p and the convergence test.
-// Over a full 3x3 block-CSR (ysp_pcg_solve_full) an iteration is two: (3) is part of (1),
-// which forms p = z + beta p_old where it reads it.
+// Over a full 3x3 block-CSR (ysp_pcg_solve_full) of up to kFuseEntries entries an iteration is
+// two: (3) is part of (1), which forms p = z + beta p_old where it reads it.
 // Scalars live in rotating sets (k mod 3) so that every kernel of iteration k reads
 // complete sums and no kernel overwrites a set another kernel of the same launch reads.
 // Each dot is a set of 64 partial-sum slots (one per 128-byte line, workgroup w adds into
@@ -455,23 +455,35 @@ __global__ void __launch_bounds__(256) direction_test_kernel(double* st, int k) 
   D.finish(st, k, threadIdx.x == 0);
 }
 
-// Kernel 1 of iteration k over the full block-CSR: the test of iteration k - 1, p = z +
-// beta p_old for the rows' own entries (stored to p) and, in registers, for every entry
-// gathered, q = A p and p^T q. The first num_long workgroups take a long row each, the
-// others 16 rows. The loop's kernels last a few microseconds each, as long as the gaps
-// between their launches: a direction kernel and a launch for the long rows of their own
-// made it four launches and 20.1 us of kernels per iteration at 11,000 rows, this makes it two
-// and 14.2 (direction, product and long rows 14.4 -> 9.6).
-template <typename Src>
+// q = A p over the full block-CSR, every row written, and p^T q into quad (if not null). The
+// first num_long workgroups take a long row each, the others 16 rows.
+//
+// kFuse: kernel 1 of iteration k, st the scalar state: the test of iteration k - 1 first, and p
+// = z + beta p_old is formed for the rows' own entries (stored to p) and, in registers, for every
+// entry gathered. Otherwise p is read as z, and *stop != 0 ends the launch.
+//
+// Small operators: the loop's kernels last a few microseconds each, as long as the gaps between
+// their launches, and the fused form takes two launches where the other takes three. Large
+// ones: it gathers two vectors per entry in place of one and forms p once per entry in place of
+// once per row. Microseconds per iteration, fused against three launches, on contact scenes:
+//   entries      33,000        397,000       674,000       1.36M         2.46M         4.47M
+//   FP64 values  11.9 / 15.2   19.6 / 20.6   26.2 / 26.6   39.5 / 36.8   62.2 / 52.6   128 / 104
+//   FP32 values  11.8 / 15.2   16.7 / 18.0   23.1 / 22.6   35.6 / 30.0   56.6 / 42.1   90 / 64
+// (the upper storage crosses at the same size: 30.5 / 30.1 at 674,000). Long rows in a launch of
+// their own and q cleared by the update cost the three-launch form 4 to 6 microseconds more.
+constexpr uint32_t kFuseEntries = 600000;
+template <bool kFuse, typename Src>
 __global__ void __launch_bounds__(kFullThreads)
-    full3_direction_kernel(const uint32_t* __restrict__ row_ptr, const uint32_t* __restrict__ col,
-                           Src vals, uint32_t nbr, uint32_t long_row,
-                           const uint32_t* __restrict__ long_rows, uint32_t num_long, int reverse,
-                           const double* __restrict__ z, const double* __restrict__ p_old,
-                           double* __restrict__ p, double* __restrict__ q,
-                           double* __restrict__ st, int k) {
-  DirectionState D;
-  D.issue(st, k);
+    full3_product_kernel(const uint32_t* __restrict__ row_ptr, const uint32_t* __restrict__ col,
+                         Src vals, uint32_t nbr, uint32_t long_row,
+                         const uint32_t* __restrict__ long_rows, uint32_t num_long, int reverse,
+                         const double* __restrict__ z, const double* __restrict__ p_old,
+                         double* __restrict__ p, double* __restrict__ q,
+                         double* __restrict__ quad, const double* __restrict__ stop,
+                         double* __restrict__ st, int k) {
+  DirectionState D{};
+  if constexpr (kFuse) D.issue(st, k);
+  else if (stop) D.status = *stop;               // written by other launches only: uniform
   const bool is_long = blockIdx.x < num_long;
   const uint32_t step = is_long ? kFullThreads : kFullLanes;
   const uint32_t l = threadIdx.x % step;
@@ -500,21 +512,30 @@ __global__ void __launch_bounds__(kFullThreads)
     z0 = z[c];
     z1 = z[c + 1];
     z2 = z[c + 2];
-    o0 = p_old[c];
-    o1 = p_old[c + 1];
-    o2 = p_old[c + 2];
+    if constexpr (kFuse) {
+      o0 = p_old[c];
+      o1 = p_old[c + 1];
+      o2 = p_old[c + 2];
+    }
     vals.load(e, b);
   };
   if (e < k1) fetch();
   const bool writes = own && l < 3;
   if (writes) {
     zr = z[3 * r + l];
-    pr = p_old[3 * r + l];
+    if constexpr (kFuse) pr = p_old[3 * r + l];
   }
-  if (!D.finish(st, k, blockIdx.x == 0 && threadIdx.x == 0)) return;
+  if constexpr (kFuse) {
+    if (!D.finish(st, k, blockIdx.x == 0 && threadIdx.x == 0)) return;
+  } else {
+    if (D.status != 0.0) return;
+  }
   double y0 = 0.0, y1 = 0.0, y2 = 0.0;
   while (e < k1) {
-    block_fma(b, z0 + o0 * D.beta, z1 + o1 * D.beta, z2 + o2 * D.beta, y0, y1, y2);
+    if constexpr (kFuse)
+      block_fma(b, z0 + o0 * D.beta, z1 + o1 * D.beta, z2 + o2 * D.beta, y0, y1, y2);
+    else
+      block_fma(b, z0, z1, z2, y0, y1, y2);
     e += step;
     if (e < k1) fetch();
   }
@@ -534,13 +555,22 @@ __global__ void __launch_bounds__(kFullThreads)
   double pq = 0.0;
   if (writes) {
     const double y = l == 0 ? y0 : (l == 1 ? y1 : y2);
-    pr = zr + pr * D.beta;
-    p[3 * r + l] = pr;
+    if constexpr (kFuse) {
+      zr = zr + pr * D.beta;
+      p[3 * r + l] = zr;
+    }
     q[3 * r + l] = y;
-    pq = pr * y;
+    pq = zr * y;
   }
-  pq = block_sum<kFullThreads>(pq, red);
-  if (threadIdx.x == 0) atomic_add_f64(my_slot(st, SET_PAP + k % 3), pq);
+  if (!quad) return;
+  // a long row's three terms sit in the first lanes of its first wavefront
+  if (is_long) {
+    if (threadIdx.x >= 64) return;
+    pq = wave_sum(pq);
+  } else {
+    pq = block_sum<kFullThreads>(pq, red);
+  }
+  if (threadIdx.x == 0) atomic_add_f64(quad + (blockIdx.x % kQuadSlots) * kQuadSpace, pq);
 }
 
 // Pinned status mailbox shared by the solves issued from this process.
@@ -605,11 +635,11 @@ extern "C" int ysp_invert_diagonal_blocks(const double* diagonal_blocks, double*
 
 namespace ysp {
 namespace {
-// The PCG loop over any operator, one of the two callables being nullptr: product(x, y, quad,
-// stop) adds A x to y, which is zero on entry, and x^T A x into the partial-sum set quad if
-// that is not null; direction(z, p_old, p, q, st, k) launches kernel 1 of the two-kernel
-// iteration, p alternating between two vectors.
-template <typename Product, typename Direction>
+// The PCG loop over any operator: product(x, y, quad, stop) forms A x in y (kAdds: adds it to y,
+// which is zero on entry) and adds x^T A x into the partial-sum set quad if that is not null;
+// direction(z, p_old, p, q, st, k), if given, launches kernel 1 of the two-kernel iteration in
+// its place, p alternating between two vectors.
+template <bool kAdds, typename Product, typename Direction>
 int generic_run(Product&& product, Direction&& direction, uint32_t max_iterations, double threshold,
                 int32_t threshold_mode, const double* diagonal_blocks_inverse,
                 const uint32_t* diagonal_blocks_start, const uint32_t* diagonal_blocks_count,
@@ -658,14 +688,8 @@ int generic_run(Product&& product, Direction&& direction, uint32_t max_iteration
   YSP_CHECK(hipMemsetAsync(st, 0, kStateDoubles * sizeof(double), s));
   const int have_guess = (!zero_initial_guess && initial_guess) ? 1 : 0;
   if (have_guess) {
-    if constexpr (kFused) {
-      // the first direction of a system whose z is the guess: p2 = x0, q = A x0
-      if (int rc = direction(initial_guess, initial_guess, p2, q, st, 1)) return rc;
-      YSP_CHECK(hipMemsetAsync(st, 0, kStateDoubles * sizeof(double), s));
-    } else {
-      YSP_CHECK(hipMemsetAsync(q, 0, sizeof(double) * n, s));
-      if (int rc = product(initial_guess, q, nullptr, nullptr)) return rc;
-    }
+    if (kAdds) YSP_CHECK(hipMemsetAsync(q, 0, sizeof(double) * n, s));
+    if (int rc = product(initial_guess, q, nullptr, nullptr)) return rc;
   }
   hipLaunchKernelGGL(init_kernel, vgrid, vblock, 0, s, L, diagonal_blocks_inverse, rhs, x,
                      initial_guess, r, p, z, q, st, have_guess);
@@ -698,7 +722,7 @@ int generic_run(Product&& product, Direction&& direction, uint32_t max_iteration
       } else {
         if (int rc = product(p, q, st + set_base(SET_PAP + cur), st + S_STATUS)) return rc;
       }
-      hipLaunchKernelGGL(update_kernel<!kFused>, vgrid, vblock, 0, s, L, diagonal_blocks_inverse, x,
+      hipLaunchKernelGGL(update_kernel<kAdds>, vgrid, vblock, 0, s, L, diagonal_blocks_inverse, x,
                          r, p, q, z, st, static_cast<int>(it));
       if constexpr (!kFused)
         hipLaunchKernelGGL(direction_kernel, dgrid, vblock, 0, s, z, p, st, n,
@@ -756,10 +780,10 @@ extern "C" int ysp_pcg_solve(uint32_t max_iterations, double threshold, int32_t 
     if (int rc = launch_part_spmv(part, x, y, 0, quad, stop, s)) return rc;
     return launch_part_spmv(dynamic_part, x, y, 0, quad, stop, s);
   };
-  return generic_run(product, nullptr, max_iterations, threshold, threshold_mode, diagonal_blocks_inverse,
-                     diagonal_blocks_start, diagonal_blocks_count, diagonal_blocks_size,
-                     gradient_segments_start, num_attributes, rhs, n, solution, initial_guess,
-                     zero_initial_guess, work, cg_scalars, stats, s);
+  return generic_run<true>(product, nullptr, max_iterations, threshold, threshold_mode,
+                           diagonal_blocks_inverse, diagonal_blocks_start, diagonal_blocks_count,
+                           diagonal_blocks_size, gradient_segments_start, num_attributes, rhs, n,
+                           solution, initial_guess, zero_initial_guess, work, cg_scalars, stats, s);
 }
 
 extern "C" int ysp_pcg_solve_full(uint32_t max_iterations, double threshold,
@@ -809,15 +833,16 @@ extern "C" int ysp_pcg_solve_full(uint32_t max_iterations, double threshold,
   int reverse = 0;                 // direction of the next product's row walk
   // value source (values.hpp): FP64 or FP32 copy (FP32 values, the mixed-precision inner
   // solve, are widened to FP64 as they are read) or the upper storage read in place
-  auto direction = [&](const double* z, const double* p_old, double* p, double* q, double* st,
-                       int k) -> int {
+  auto launch = [&](auto fuse, const double* z, const double* p_old, double* p, double* q,
+                    double* quad, const double* stop, double* st, int k) -> int {
     if (int rc = with_values(values, values_f32, nnz, "ysp_pcg_solve_full: bad value source",
                              [&](auto vals) {
-                               hipLaunchKernelGGL(full3_direction_kernel<decltype(vals)>,
+                               hipLaunchKernelGGL((full3_product_kernel<decltype(fuse)::value,
+                                                                        decltype(vals)>),
                                                   dim3(num_long_rows + grid_for(nbr, kFullRows)),
                                                   dim3(kFullThreads), 0, s, row_ptr, col, vals,
                                                   nbr, long_row, long_rows, num_long_rows, reverse,
-                                                  z, p_old, p, q, st, k);
+                                                  z, p_old, p, q, quad, stop, st, k);
                                return YSP_OK;
                              }))
       return rc;
@@ -825,8 +850,18 @@ extern "C" int ysp_pcg_solve_full(uint32_t max_iterations, double threshold,
     YSP_CHECK_LAUNCH();
     return YSP_OK;
   };
-  return generic_run(nullptr, direction, max_iterations, threshold, threshold_mode, diagonal_blocks_inverse,
-                     diagonal_blocks_start, diagonal_blocks_count, diagonal_blocks_size,
-                     gradient_segments_start, num_attributes, rhs, n, solution, initial_guess,
-                     zero_initial_guess, work, cg_scalars, stats, s);
+  auto product = [&](const double* x, double* y, double* quad, const double* stop) -> int {
+    return launch(std::false_type(), x, nullptr, nullptr, y, quad, stop, nullptr, 0);
+  };
+  auto direction = [&](const double* z, const double* p_old, double* p, double* q, double* st,
+                       int k) -> int {
+    return launch(std::true_type(), z, p_old, p, q, st + set_base(SET_PAP + k % 3), nullptr, st, k);
+  };
+  auto run = [&](auto&& dir) {
+    return generic_run<false>(product, dir, max_iterations, threshold, threshold_mode,
+                              diagonal_blocks_inverse, diagonal_blocks_start, diagonal_blocks_count,
+                              diagonal_blocks_size, gradient_segments_start, num_attributes, rhs, n,
+                              solution, initial_guess, zero_initial_guess, work, cg_scalars, stats, s);
+  };
+  return nnz <= kFuseEntries ? run(direction) : run(nullptr);
 }
