@@ -8,7 +8,13 @@
 // Layout: row_ptr[nbr + 1], col[nnz] (block column), src[nnz] (bit 31: stored
 // transposed, bit 30: dynamic part, low bits: upper block index) and component-major
 // values v[j * stride + k] (j = 0..8 row-major entry of block k, stride = nnz rounded up
-// to 64) so that 16 lanes reading 16 consecutive blocks issue fully coalesced loads.
+// to 64) so that 16 lanes reading 16 consecutive blocks issue fully coalesced loads. Each
+// row is summed in a fixed order.
+//
+// The block-Jacobi PCG of large static operators reads a tiled symmetric copy instead
+// (tiles.hpp). Its rows are summed through LDS atomics, in an order that follows the
+// schedule: its products agree with the mirrored ones to rounding, not bit for bit, and
+// neither do two of its own.
 #include "common.hpp"
 #include "dense.hpp"
 #include "mas.hpp"

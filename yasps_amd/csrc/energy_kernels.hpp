@@ -211,14 +211,15 @@ __device__ __forceinline__ double hget(const double (&H)[N * (N + 1) / 2], int i
 // entry serialises on a few addresses. Blocks coupling two affine groups and gradient
 // segments of affine groups are summed in LDS instead (a few slots keyed by the
 // destination's offset, found by all, with a sum for each wavefront) and leave with one
-// global atomic per entry and workgroup, the wavefronts' sums added in order: a list that
-// one workgroup takes gives the same bits every time. A destination that finds no free slot
-// takes the global atomic directly.
+// global atomic per entry and workgroup, the wavefronts' sums added in order. A destination
+// that finds no free slot takes the global atomic directly. The assembled bits are not
+// reproducible: the list's order past one evaluation wavefront, which destinations find a
+// slot when there are more than slots, and every global atomic follow the schedule.
 constexpr unsigned kGB = 1024, kGW = kGB / 64;
-// Lists up to this length go to one workgroup: small scenes, whose other sums one wavefront
-// forms, are then assembled to the same bits every time (a stiff solve's iteration count
-// depends on them). Longer ones are spread over the chip: with 256 elements a workgroup
-// 7,000 tets and 42,000 pairs took 344 us each, spread 64.
+// Lists up to this length go to one workgroup: fewer sums depend on the schedule then (spread
+// over workgroups, the iteration counts of two solves of a small stiff scene differed in 5 of 25
+// pairs, in one workgroup in none; no guarantee, see above). Longer ones are spread over the
+// chip: with 256 elements a workgroup 7,000 tets and 42,000 pairs took 344 us each, spread 64.
 constexpr uint32_t kGRun = 256;
 constexpr uint32_t kHotEmpty = 0xffffffffu;
 constexpr int kHotBlocks = 8, kHotBlockMax = 81, kHotGrad = 4, kHotGradMax = 9;
