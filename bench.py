@@ -62,13 +62,13 @@ def parse():
     return ap.parse_args()
 
 
-# the PCG product kernel on the mirrored FP64 copy, as rocprofv3 names it
-PRODUCT_KERNEL = "pcg3_spmv_kernel<ysp::Mirrored<double>"
+# the PCG product kernels (the tiled operator of large static systems, the mirrored FP64 copy), as
+# rocprofv3 names them
+PRODUCT_KERNELS = ("pcg3_tiled_kernel<double>", "pcg3_spmv_kernel<ysp::Mirrored<double>")
 
 
 def measure_traffic(args):
-    """HBM bytes per launch of pcg3_spmv_kernel<Mirrored<double>> (the PCG loop's product kernel) from
-    two hardware-counter runs, FETCH_SIZE then WRITE_SIZE, of ``bench.py --kernels-only``
+    """HBM bytes per launch of the PCG loop's product kernel from two hardware-counter runs, FETCH_SIZE then WRITE_SIZE, of ``bench.py --kernels-only``
     under rocprofv3, each counter scaled by its reading for a 256 MiB device copy of known
     size. Runs as child processes before this process touches the GPU. Returns
     (bytes, details); bytes is None when the counters could not be collected."""
@@ -107,7 +107,7 @@ def measure_traffic(args):
                         if row.get("Counter_Name") != counter:
                             continue
                         name = row.get("Kernel_Name", "")
-                        if PRODUCT_KERNEL in name:
+                        if any(k in name for k in PRODUCT_KERNELS):
                             prod.append(float(row["Counter_Value"]))
                         elif "copyBuffer" in name:
                             copy.append(float(row["Counter_Value"]))
@@ -139,18 +139,20 @@ def calibration_copy(mib=256):
 
 
 def product_roofline(hs, reps, traffic=None, traffic_detail=None, cold_reps=20, replicas=4):
-    """Roofline of pcg3_spmv_kernel<Mirrored<double>>, the kernel that dominates the timed PCG loop
-    (one launch per iteration: q = A z + beta q, p = z + beta p and the partial sums of
-    p.q over the mirrored 3x3 block-CSR), launched through ysp_pcg3_product_pass with the
-    loop's own grid and timed by HIP events on the stream it runs on.
+    """Roofline of the product kernel of the timed PCG loop (one launch per iteration:
+    q = A z + beta q, p = z + beta p and the partial sums of p.q), on the operator that the
+    loop reads (``hs.pcg_values``: the tiled symmetric copy at n=48, pcg3_tiled_kernel<double>;
+    the mirrored 3x3 block-CSR below its size, pcg3_spmv_kernel<Mirrored<double>>), launched
+    through ysp_pcg3_product_pass with the loop's own grid and timed by HIP events on the
+    stream it runs on.
 
     Algorithmic bytes per launch: the upper 3x3 blocks read once (72 B values + 8 B (row,
     col)) plus five vector passes (z read, p read and written, q read and written). Two
     regimes, each a run of back-to-back launches between one pair of events:
-    * in the loop: launches on one operator, which (134 MB at n=48) then stays in the
+    * in the loop: launches on one operator, which (100 MB at n=48) then stays in the
       256 MB Infinity Cache;
     * HBM (the headline): launches rotating over ``replicas`` copies of the operator and of
-      the vectors (4 x 155 MB at n=48), so that each launch finds its operands evicted by
+      the vectors (4 x 100 MB at n=48), so that each launch finds its operands evicted by
       the launches on the other copies and streams them from HBM."""
     from yasps_amd import _lib, device as dev
     torch = dev.torch()
@@ -158,16 +160,21 @@ def product_roofline(hs, reps, traffic=None, traffic_detail=None, cold_reps=20, 
     f = hs.full
     n = hs.rows
     stream = torch.cuda.current_stream()
+    tl = f.tiles if hs.pcg_values()[1] == _lib.VALUES_TILED else None
 
     def make(copy):
-        if not copy:
-            return (f.row_ptr, f.col, f.v64, dev.zeros(5 * n, "float64"), dev.zeros(12288, "float64"))
-        return (f.row_ptr.clone(), f.col.clone(), f.v64.clone(), dev.zeros(5 * n, "float64"),
-                dev.zeros(12288, "float64"))           # 12288 = YSP_PCG3_SCALARS
+        state = (dev.zeros(5 * n, "float64"), dev.zeros(12288, "float64"))   # YSP_PCG3_SCALARS
+        c = (lambda t: t.clone()) if copy else (lambda t: t)
+        if tl is None:
+            v = c(f.v64)
+            return (c(f.row_ptr), c(f.col), v, dev.ptr(v), 0, *state)
+        held = [c(t) for t in (tl.rows, tl.lens, tl.slice_start, tl.entry, tl.v64)]
+        d = _lib.TiledValues(*map(dev.ptr, held[:4]), tl.entries, dev.ptr(held[4]), 0)
+        return (f.row_ptr, f.col, (held, d), C.addressof(d), _lib.VALUES_TILED, *state)
 
     def launch(op, prepare=0):
-        rp, col, v, work, scal = op
-        _lib.check(lib.ysp_pcg3_product_pass(dev.ptr(rp), dev.ptr(col), dev.ptr(v), 0, f.nnz, n,
+        rp, col, _, v, fmt, work, scal = op
+        _lib.check(lib.ysp_pcg3_product_pass(dev.ptr(rp), dev.ptr(col), v, fmt, f.nnz, n,
                                              dev.ptr(work), dev.ptr(scal), prepare,
                                              stream.cuda_stream), "ysp_pcg3_product_pass")
 
@@ -198,24 +205,24 @@ def product_roofline(hs, reps, traffic=None, traffic_detail=None, cold_reps=20, 
     del ops
     nb = hs.static.num_blocks
     bytes_alg = nb * (9 * 8 + 8) + 5 * n * 8
-    bytes_full = f.nnz * (9 * 8 + 4) + (n // 3 + 1) * 4 + 5 * n * 8
+    # what the layout holds: values and column of every entry, row lengths or starts, vectors
+    bytes_full = (tl.entries if tl else f.nnz) * (9 * 8 + 4) + (n // 3 + 1) * 4 + 5 * n * 8
     gbs_cold = bytes_alg / (ms_cold * 1e-3) / 1e9
     gbs_warm = bytes_alg / (ms_warm * 1e-3) / 1e9
     return {"bound": "hbm", "achieved": round(gbs_cold, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(gbs_cold / HBM_PEAK_GBS, 4), "traffic": traffic,
-            "kernel": "pcg3_spmv_kernel<Mirrored<double>>",
+            "kernel": "pcg3_tiled_kernel<double>" if tl else "pcg3_spmv_kernel<Mirrored<double>>",
             "regime": (f"HBM: back-to-back launches rotating over {replicas} copies of the "
                        "operator and vectors (each launch streams its operands from HBM)"),
             "avg_us": round(ms_cold * 1e3, 2), "launches": cold_reps * replicas if cold_reps else 0,
-            "bytes_per_launch": int(bytes_alg), "full_bsr_bytes_per_launch": int(bytes_full),
-            "full_bsr_GBs": round(bytes_full / (ms_cold * 1e-3) / 1e9, 1),
+            "bytes_per_launch": int(bytes_alg), "layout_bytes_per_launch": int(bytes_full),
+            "layout_GBs": round(bytes_full / (ms_cold * 1e-3) / 1e9, 1),
             "in_loop": {"avg_us": round(ms_warm * 1e3, 2), "launches": reps,
                         "achieved": round(gbs_warm, 1),
                         "frac": round(gbs_warm / HBM_PEAK_GBS, 4),
-                        "full_bsr_GBs": round(bytes_full / (ms_warm * 1e-3) / 1e9, 1),
+                        "layout_GBs": round(bytes_full / (ms_warm * 1e-3) / 1e9, 1),
                         "note": ("back-to-back launches on one operator as in the PCG loop: "
-                                 "the operator (134 MB at n=48) stays in the 256 MB Infinity "
-                                 "Cache")},
+                                 "the operator stays in the 256 MB Infinity Cache at n=48")},
             "traffic_detail": traffic_detail}
 
 
@@ -829,7 +836,7 @@ def main():
     if args.kernels_only:
         # assembly only (the operator of the loop), then the product launches (back to back
         # on one operator, then rotating over its copies) and the calibration copy: the only
-        # pcg3_spmv_kernel launches are the measured ones
+        # product launches are the measured ones
         s0.minimizer.computeNumericValue()
         roof = product_roofline(s0.minimizer.activeHessian, args.spmv_reps,
                                 cold_reps=args.cold_reps)

@@ -642,7 +642,8 @@ int ysp_pcg3_mas_solve(uint32_t max_iterations, double threshold, int32_t thresh
  * prepare != 0 the scalar state is first set to a running iteration (beta = 1, never
  * converged) and z, p, q to nonzero data; later passes keep updating p and q. Every block
  * row goes through the product kernel (no long-row list). work: 5 n doubles laid out as
- * ysp_pcg3_solve's, cg_scalars: YSP_PCG3_SCALARS doubles. Asynchronous. */
+ * ysp_pcg3_solve's (in tile order with YSP_VALUES_TILED), cg_scalars: YSP_PCG3_SCALARS doubles.
+ * Asynchronous. */
 int ysp_pcg3_product_pass(const uint32_t* row_ptr, const uint32_t* col, const void* values,
                           int32_t values_f32, uint32_t nnz, uint32_t n, double* work,
                           double* cg_scalars, int32_t prepare, void* stream);

@@ -1631,16 +1631,21 @@ extern "C" int ysp_pcg3_product_pass(const uint32_t* row_ptr, const uint32_t* co
     hipLaunchKernelGGL(product_state_kernel, dim3(grid_for(n, kB)), dim3(kB), 0, s, cg_scalars,
                        z, pa, q, n);
   }
-  const uint32_t rows_per_wg = spmv_rows_per_wg(nv);
-  const dim3 sg(grid_for(nv, rows_per_wg)), bl(kB);
-  return with_values(values, values_f32, nnz, "ysp_pcg3_product_pass: bad value source",
-                     [&](auto vals) {
-                       hipLaunchKernelGGL(pcg3_spmv_kernel<decltype(vals)>, sg, bl, 0, s, row_ptr,
-                                          col, vals, nv, z, pa, q, cg_scalars, 2, rows_per_wg,
-                                          nullptr, nullptr, nullptr, 0);
-                       YSP_CHECK_LAUNCH();
-                       return YSP_OK;
-                     });
+  return with_pcg_values(values, values_f32, nnz, "ysp_pcg3_product_pass: bad value source",
+                         [&](auto vals) {
+    using Src = decltype(vals);
+    if constexpr (is_tiled<Src>::value) {
+      hipLaunchKernelGGL(pcg3_tiled_kernel, dim3(grid_for(nv, kTileRows)), dim3(kTileThreads), 0, s,
+                         vals, nv, z, pa, q, cg_scalars, 2, 0);
+    } else {
+      const uint32_t rows_per_wg = spmv_rows_per_wg(nv);
+      hipLaunchKernelGGL(pcg3_spmv_kernel<Src>, dim3(grid_for(nv, rows_per_wg)), dim3(kB), 0, s,
+                         row_ptr, col, vals, nv, z, pa, q, cg_scalars, 2, rows_per_wg, nullptr,
+                         nullptr, nullptr, 0);
+    }
+    YSP_CHECK_LAUNCH();
+    return YSP_OK;
+  });
 }
 
 // ---------------------------------------------------------- PCG without allocations
