@@ -31,21 +31,38 @@ def system():
     return s0, hs, H, M, dev.to_host(hs.gradient.value)
 
 
-def _solve(hs, max_it, tol, guess=None, long_row=0, sign=1.0):
+def _solve(hs, max_it, tol, guess=None, long_row=0, sign=1.0, source="f64"):
     from yasps_amd import _lib, device as dev
     f, n = hs.split, hs.rows
     x, work, scalars = dev.zeros(n, "float64"), dev.zeros(5 * n, "float64"), dev.zeros(12288, "float64")
-    values = f.v64 * sign
+    held = f.v64 * sign if source == "f64" else hs.full_values_f32()
+    values, fmt = dev.ptr(held), int(source == "f32")
+    if source == "upper":
+        hs.value_source = "upper"
+        values, fmt = hs.solve_values()
+        hs.value_source = "auto"
     st = _lib.PcgStats()
     g = None if guess is None else dev.to_device(guess, "float64")
     rc = _lib.load().ysp_pcg_solve_full(
-        max_it, tol, 1, dev.ptr(f.row_ptr), dev.ptr(f.col), dev.ptr(values), 0, f.nnz, long_row,
+        max_it, tol, 1, dev.ptr(f.row_ptr), dev.ptr(f.col), values, fmt, f.nnz, long_row,
         dev.ptr(hs.diagonal_blocks_inverse), _lib.u32_array(hs.diagonal_blocks_start_cpu[:-1]),
         _lib.u32_array([w.numInstances for w in hs.wrt]), _lib.u32_array([w.size for w in hs.wrt]),
         _lib.u32_array(hs.gradient_segments_start_cpu[:-1]), len(hs.wrt),
         dev.ptr(hs.gradient.value), n, dev.ptr(x), dev.ptr(g), int(g is None), dev.ptr(work),
         dev.ptr(scalars), C.byref(st), dev.stream())
     return rc, st, dev.to_host(x)
+
+
+def _rounded(hs):
+    """The operator with every entry of the split block-CSR rounded to FP32 (a block of the
+    static and one of the dynamic part at the same place are entries of their own)."""
+    from yasps_amd import device as dev
+    f, A = hs.split, np.zeros((hs.rows // 3, 3, hs.rows // 3, 3))
+    v = dev.to_host(f.v64).reshape(9, -1)[:, :f.nnz].T.reshape(-1, 3, 3)
+    row = np.repeat(np.arange(f.nbr), np.diff(dev.to_host(f.row_ptr, "uint32").astype(np.int64)))
+    np.add.at(A, (row, slice(None), dev.to_host(f.col, "uint32")[:f.nnz].astype(np.int64)),
+              v.astype(np.float32).astype(np.float64))
+    return A.reshape(hs.rows, hs.rows)
 
 
 def _pcg(H, M, b, x, iterations):
@@ -74,6 +91,20 @@ def test_iterates(system, max_it, long_row):
         # rounding of a dot or product (1e-14 here), amplified by the recurrence: 1e-11 after 5
         # iterations is the bound of the long-row test, a factor 10 for the 13 here
         assert np.linalg.norm(x - want) <= 1e-10 * np.linalg.norm(want)
+        assert abs(st.delta - rz) <= 1e-8 * rz and abs(st.rr - rr) <= 1e-8 * rr
+
+
+@pytest.mark.parametrize("source", ["f32", "upper"])
+@pytest.mark.parametrize("long_row", [0, 4])
+def test_iterates_from_other_values(system, long_row, source):
+    _, hs, H, M, b = system
+    A = _rounded(hs) if source == "f32" else H
+    for max_it in (1, 5, 13):
+        print(f"{max_it} iterations, long rows from {long_row}, {source}", flush=True)
+        rc, st, x = _solve(hs, max_it, 1e-30, None, long_row, source=source)
+        want, rz, rr = _pcg(A, M, b, np.zeros_like(b), max_it)
+        assert rc == -4 and st.iterations == max_it
+        assert np.linalg.norm(x - want) <= 1e-10 * np.linalg.norm(want)      # as above
         assert abs(st.delta - rz) <= 1e-8 * rz and abs(st.rr - rr) <= 1e-8 * rr
 
 

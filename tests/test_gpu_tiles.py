@@ -141,7 +141,7 @@ def test_rows_too_long_for_tiles_are_refused():
 
 def test_scene_uses_tiles_and_matches_mirrored():
     """A cube above the size from which the solver reads tiles, against the mirrored copy."""
-    from yasps_amd import device as dev
+    from yasps_amd import _lib, device as dev
     from yasps_amd.scenes import cube_scene, build_yasps_scene
     print("tiles: n=32 cube", flush=True)
     x = {}
@@ -151,4 +151,57 @@ def test_scene_uses_tiles_and_matches_mirrored():
         h.value_source = source
         assert (h.full.tiles is not None) and h.full.tiles.entries < 0.9 * h.full.nnz
         x[source] = dev.to_host(s0.minimizeEnergy(tolerance=1e-10)[0]).copy()
+        # what the solve read
+        tiled = source == "auto"
+        assert h.pcg_values()[1] == (_lib.VALUES_TILED if tiled else _lib.VALUES_F64)
+        assert h.full.tiles.valid64 == tiled and not h.full.tiles.valid32
     assert np.linalg.norm(x["auto"] - x["mirrored"]) <= 1e-8 * np.linalg.norm(x["mirrored"])
+
+
+def test_mixed_solve_through_tiles():
+    """FP32 tiles in the Krylov loop, FP64 refinement: the true residual, and the FP64
+    solution to the tolerance times the condition of the cube (below 1e3)."""
+    from yasps_amd import _lib, device as dev
+    from yasps_amd.hessian import vector
+    from yasps_amd.scenes import cube_scene, build_yasps_scene
+    print("tiles: n=32 cube, mixed", flush=True)
+    x = {}
+    for precision in ("fp64", "mixed"):
+        s0, _ = build_yasps_scene(cube_scene(32, seed=1), threshold_mode="relative_residual",
+                                  precision=precision)
+        x[precision] = s0.minimizeEnergy(tolerance=1e-10)[0].reshape(-1).clone()
+        h = s0.minimizer.activeHessian
+        mixed = precision == "mixed"
+        assert h.pcg_values(f32=mixed)[1] == _lib.VALUES_TILED
+        assert h.full.tiles.valid32 == mixed and h.full.tiles.valid64 == (not mixed)
+        g = h.gradient.value
+        r = h.spmv(vector(h.rows, x[precision].clone())).value - g
+        assert float(r.norm() / g.norm()) <= 1.01e-10
+    assert float((x["mixed"] - x["fp64"]).norm() / x["fp64"].norm()) <= 1e-7
+
+
+def test_product_pass_over_tiles():
+    """One pass of the loop's product on prepared state: p = z + p0, q = A z + q0 in tile order."""
+    from yasps_amd import _lib, device as dev
+    from yasps_amd.hessian import vector
+    from yasps_amd.scenes import cube_scene, build_yasps_scene
+    print("tiles: product pass", flush=True)
+    s0, _ = build_yasps_scene(cube_scene(32, seed=1))
+    h = s0.minimizer.computeNumericValue()
+    n, f = h.rows, h.full
+    values, fmt = h.pcg_values()
+    assert fmt == _lib.VALUES_TILED
+    work, scalars = dev.zeros(5 * n, "float64"), dev.zeros(12288, "float64")
+    _lib.check(_lib.load().ysp_pcg3_product_pass(
+        dev.ptr(f.row_ptr), dev.ptr(f.col), values, fmt, f.nnz, n, dev.ptr(work), dev.ptr(scalars), 1,
+        dev.stream()), "ysp_pcg3_product_pass")
+    z, p, q = (dev.to_host(work)[k * n:(k + 1) * n] for k in (1, 2, 4))
+    assert np.array_equal(z, 1.0 + 0.01 * (np.arange(n) % 7)) and np.array_equal(p, z + 0.5)
+    rows = dev.to_host(f.tiles.rows, "uint32").astype(np.int64)
+    order = (3 * rows[:, None] + np.arange(3)).ravel()
+    zn = np.empty(n)
+    zn[order] = z
+    want = h.spmv(vector().updateValue(zn)).get()[order] + 0.25
+    # sums of at most 96 entries in another order: 96 x 3 eps of the largest product
+    scale = np.abs(dev.to_host(h.blocks_flattened)).max() * np.abs(z).max()
+    assert np.abs(q - want).max() <= 288 * np.finfo(np.float64).eps * scale * 3
