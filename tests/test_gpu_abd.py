@@ -122,3 +122,42 @@ def test_abd_index_pipeline_bit_exact():
     assert hs.static.dims == layout.block_dimensions
     for ti, lk in zip(hs.static_index, layout.lookups):
         np.testing.assert_array_equal(dev.to_host(ti.lookups, "uint32"), lk)
+
+
+@pytest.mark.parametrize("method", [0, 1, 2])
+def test_point_pairs_on_affine_bodies(method):
+    """6 x 6 Hessians, projected where they are evaluated, of pairs whose points are affine,
+    free and fixed vertices: the general scatter's blocks against the chain rule over the
+    oracle's projected pairs."""
+    from oracle import element_energies as oe, projection
+    from yasps_amd import device as dev
+    from yasps_amd.energies import point_point
+    print(f"point pairs on affine bodies, method {method}", flush=True)
+    sc = abd_cube_scene(n=3, abd_layers=2, bodies=2, seed=3)
+    s0, hd = build_abd_scene(sc, projection_method=method)
+    base = s0.minimizer.computeNumericValue()
+    g0, H0 = dev.to_host(base.gradient.value).copy(), np.asarray(base.dense())
+    nv = sc.cube.rest.shape[0]
+    rng = np.random.default_rng(0)
+    pairs = np.array([rng.choice(nv, 2, replace=False) for _ in range(300)], dtype=np.uint32)
+    s0, hd = build_abd_scene(sc, projection_method=method)
+    m = hd["mesh"]
+    el = m.addPrimitive("pairs", numInstances=len(pairs))
+    e2v = el.addConnectivity("pairs2v", m.vertices, pairs, 2)
+    p = el.addAttribute("positions", through=e2v, source=m.vertices["position"])
+    dhat, kappa = 4.0, 1e-2                              # every pair of the unit cube is active
+    s0.addEnergy(el.addAttribute("pp", computed_attribute=point_point(p, dhat, kappa)),
+                 projection_method=method)
+    hs = s0.minimizer.computeNumericValue()
+    g, H = dev.to_host(hs.gradient.value), np.asarray(hs.dense())
+    X = sc.positions()[pairs.astype(np.int64)].reshape(-1, 6)
+    _, ge, He = oe.evaluate("point_point", X, np.zeros((len(pairs), 0)), np.array([dhat, kappa]))
+    want_g, want_H = g0.copy(), H0.copy()
+    for k, (a, b) in enumerate(pairs):
+        Hk = projection.project(He[k], method) if method else He[k]
+        ends = [abd.vertex_jacobian(sc, int(v)) for v in (a, b)]
+        for i, (di, Ji) in enumerate(ends):
+            want_g[di] += Ji.T @ ge[k][3 * i:3 * i + 3]
+            for j, (dj, Jj) in enumerate(ends):
+                want_H[np.ix_(di, dj)] += Ji.T @ Hk[3 * i:3 * i + 3, 3 * j:3 * j + 3] @ Jj
+    assert _rel(g, want_g) < REL and _rel(H, want_H) < REL

@@ -721,7 +721,17 @@ __device__ __forceinline__ void scatter_vertex_blocks(const ScatterArgs& S, uint
 // Evaluation of elements [first, last): gradient and Hessian, PSD test, scatter of what
 // needs nothing else. The projection lives in a kernel of its own (below): with the
 // eigensolver inlined behind the generated code every kind's kernel held both register
-// sets and two copies of the scatter.
+// sets and two copies of the scatter. Hessians of up to kProjectInline rows are projected in
+// place all the same: 600,000 indefinite point pairs (6 x 6) took 311 us staged and 539 us with
+// atomics when they were held, 175 and 398 us in place (one kernel with Jacobi sweeps and
+// without the scatter through LDS: 210 and 1,313). The next size, 9 x 9 (point to edge), is
+// better held: 613 us against 781 in one kernel.
+constexpr int kProjectInline = 6;
+template <int ID>
+__host__ __device__ constexpr bool projects_later() {
+  return ID != YSP_ENERGY_QUADRATIC_FORM && Kind<ID>::N > kProjectInline;
+}
+
 template <int ID, int KT>
 __global__ void __launch_bounds__(kEB)
     energy_eval_kernel(UnionView P, const uint32_t* __restrict__ e2v, uint32_t first, uint32_t last,
@@ -747,7 +757,10 @@ __global__ void __launch_bounds__(kEB)
   element_eval<ID>(x, p, sp, method, E, g, H);
   bool psd = true;
   if constexpr (ID != YSP_ENERGY_QUADRATIC_FORM)
-    if (method != 0) psd = is_psd<T::N>(H);
+    if (method != 0) {
+      if constexpr (projects_later<ID>()) psd = is_psd<T::N>(H);
+      else project_packed<T::N>(H, method);
+    }
   const bool vertex = live && vs.ok, done = vertex && psd;
   scatter_vertex_gradient<T::A, T::W, T::N>(SA, e, vertex, vs, g, ws);
   scatter_vertex_blocks<T::A, T::W>(SA, e, done, vs, ws, [&](int a, int b, double (&B)[T::W][T::W]) {
@@ -892,10 +905,12 @@ int launch_eval(const UnionView& U, const AffineView& AF, const uint32_t* e2v, u
       const dim3 g(grid_for(m, kEB)), b(kEB);
       hipLaunchKernelGGL((energy_eval_kernel<ID, KT>), g, b, 0, s, U, e2v, first, first + m, ep, sp,
                          method, SA, flags, held);
-      if (method != 0 && ID != YSP_ENERGY_QUADRATIC_FORM)
-        hipLaunchKernelGGL((energy_project_kernel<T::A, T::W, KT, (translation_free<ID>() && T::A == 4 &&
-                                                                   T::W == 3)>),
-                           g, b, 0, s, method, SA, held);
+      if constexpr (projects_later<ID>()) {
+        if (method != 0)
+          hipLaunchKernelGGL((energy_project_kernel<T::A, T::W, KT, (translation_free<ID>() &&
+                                                                     T::A == 4 && T::W == 3)>),
+                             g, b, 0, s, method, SA, held);
+      }
       // usually nothing to do, or everything that an affine body drives
       hipLaunchKernelGGL((energy_scatter_kernel<T::A, T::W, KT>),
                          dim3(std::min<unsigned>(grid_for(m, kGW), AF.mask ? 256 : 64)), dim3(kGB),
