@@ -580,7 +580,7 @@ typedef struct ysp_tiled_values {
   const uint32_t* lens;
   const uint32_t* slice_start;
   const uint32_t* entry;
-  uint32_t entries;
+  uint32_t entries;                  /* as ysp_bsr3_tiles_layout returned it (not read) */
   const void* values;
   int32_t values_f32;
 } ysp_tiled_values;

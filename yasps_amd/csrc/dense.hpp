@@ -123,13 +123,13 @@ __device__ __forceinline__ double rsqrt_pos(double x) {
 //
 // One matrix per lane, every index a compile-time constant and no control flow inside a
 // sweep (a branch around each rotation made the compiler copy V at every merge, as many
-// moves as multiply-adds). Bound by FP64 VALU work and its dependent chains at one
-// wavefront per SIMD: SNH tets take 79 rotations each, about 117 with the wavefront's lanes
-// waiting for the slowest at every eigenvalue, each 36 multiply-adds on V, about 35 on
-// the tridiagonal and one reciprocal square root. The round-robin Jacobi it replaces took
-// 5.6 sweeps of 36 rotations: the projection of the 37^3-cell cube's 173,000 indefinite
-// tets 256 -> 116 us, of a 48^3-cell cube's 378,000 tets 502 -> 206 us, of one wavefront
-// 71 -> 38 us.
+// moves as multiply-adds). Bound by FP64 VALU work and its dependent chains at two
+// wavefronts per SIMD (254 VGPRs): SNH tets take 79 rotations each, about 117 with the
+// wavefront's lanes waiting for the slowest at every eigenvalue, each 36 multiply-adds on V,
+// about 35 on the tridiagonal and one reciprocal square root. The round-robin Jacobi it
+// replaces took 5.6 sweeps of 36 rotations: the projection of the 37^3-cell cube's 173,000
+// indefinite tets 256 -> 116 us, of a 48^3-cell cube's 378,000 tets 502 -> 206 us, of one
+// wavefront 71 -> 38 us.
 template <int N>
 __device__ __forceinline__ void sym_eigen_packed(double (&a)[N * (N + 1) / 2], double (&d)[N],
                                                  double (&V)[N][N]) {

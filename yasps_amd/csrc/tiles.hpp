@@ -23,7 +23,6 @@ struct TiledView {
   const uint32_t* slice_start;  // [slices + 1] first entry of each slice of 64 positions
   const uint32_t* entry;        // [entries] the column's position: in the tile, or
                                 // kTileCut | its position in the operator
-  uint32_t entries;             // including the slices' padding
 };
 
 template <typename VT>

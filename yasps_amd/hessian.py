@@ -255,8 +255,10 @@ class hessian:
         self.full: Optional[FullBsr] = None
         self.split: Optional[FullBsr] = None     # 3x3 sub-blocks of 9x9 / 9x3 / 3x9 layouts
         self.want_f32 = False
-        # where the solve loop reads FP64 operator values: "auto" (the upper storage when
-        # the mirrored copy would not stay in the Infinity Cache), "mirrored" or "upper"
+        # where the solve loop reads FP64 operator values: "auto" (block-Jacobi PCG: the tiled
+        # symmetric copy where the layout has one, see pcg_values; otherwise the upper
+        # storage when the mirrored copy would not stay in the Infinity Cache, else the
+        # mirrored copy), "mirrored" or "upper"
         self.value_source = "auto"
         self._upper = None
         self._tiled = None
@@ -666,8 +668,9 @@ class hessian:
     UPPER_VALUE_BYTES = 160 << 20
 
     def solve_values(self):
-        """(pointer, format) of the FP64 operator values the solve loop reads: the
-        component-major mirrored copy (``YSP_VALUES_F64``) or the upper block storage read
+        """(pointer, format) of the FP64 operator values that the loops read which do not take
+        the tiled operator (MAS, the split operator, systems without tiles; the block-Jacobi
+        PCG asks ``pcg_values``): the component-major mirrored copy (``YSP_VALUES_F64``) or the upper block storage read
         through each entry's source word (``YSP_VALUES_UPPER``, a ``ysp_upper_values`` held
         by this object), chosen by ``value_source``. Both give the same products."""
         f = self.operator
