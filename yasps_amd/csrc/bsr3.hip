@@ -1543,7 +1543,7 @@ int with_pcg_values(const void* values, int32_t format, uint32_t nnz, const char
     ysp_set_error(__FILE__, __LINE__, who);
     return YSP_ERR_ARG;
   }
-  const TiledView v{t->rows, t->lens, t->slice_start, t->entry};
+  const TiledView v{t->rows, t->lens, t->slice_start, t->entry, t->entries};
   if (t->values_f32) return f(Tiled<float>{v, static_cast<const float*>(t->values)});
   return f(Tiled<double>{v, static_cast<const double*>(t->values)});
 }

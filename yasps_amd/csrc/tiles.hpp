@@ -23,6 +23,9 @@ struct TiledView {
   const uint32_t* slice_start;  // [slices + 1] first entry of each slice of 64 positions
   const uint32_t* entry;        // [entries] the column's position: in the tile, or
                                 // kTileCut | its position in the operator
+  uint32_t entries;             // including the slices' padding (read by nothing; without it the
+                                // product kernel is scheduled worse: a 64^3-cell cube's solve
+                                // 10.24 -> 10.30 ms)
 };
 
 template <typename VT>
