@@ -596,8 +596,9 @@ struct TileRow {
 // pcg3_spmv_kernel over the tiled operator (same recurrence, tests and scalar state), z, p
 // and q in tile order (in the caller's order their scattered 24-byte pieces were 40% of the
 // L1 accesses: 22.1 against 18.4 us). Bound by the bytes: 48^3-cell cube 1.12M entries of 76
-// bytes and five vectors, 100 MB in 17.6 us, 5.7 TB/s where plain reads of resident data
-// reach 6.8 (mirrored 148 MB in 23.8 us); 64^3 cells 40.7 us (upper storage in place 45.3).
+// bytes and five vectors, 106 MB (hardware counters) in 17.6 us, 6.0 TB/s where plain reads of
+// resident data reach 6.8 (mirrored 148 MB in 23.8 us); 64^3 cells 40.7 us (upper storage in place
+// 45.3).
 // 512 threads at 100 VGPRs put two tiles on a compute unit; one entry per thread and group
 // measured 17.6, two 18.6, more wavefronts by spilling 30 us; tiles of 512 rows 17.0 / 44.9
 // us, of 128 rows 19.8 / 41.7 (48^3 / 64^3 cells).
