@@ -39,13 +39,14 @@ def _tets(n, seed):
 @pytest.mark.parametrize("scene,sizes", [(_membranes, (200_000, 300)), (_membranes, (300, 200_000)),
                                          (_membranes, (20_000, 20_000)), (_tets, (32, 4)),
                                          (_tets, (4, 32)), (_tets, (16, 16))])
-def test_two_streams_keep_their_hessians(scene, sizes):
+@pytest.mark.parametrize("default", [False, True])
+def test_two_streams_keep_their_hessians(scene, sizes, default):
     from yasps_amd import device as dev
     t = dev.torch()
-    print(f"element streams {scene.__name__} {sizes}", flush=True)
+    print(f"element streams {scene.__name__} {sizes} default {default}", flush=True)
     hs = [scene(n, k) for k, n in enumerate(sizes)]
     want = [(h.gradient.value.clone(), h.blocks_flattened.clone()) for h in hs]
-    streams = [t.cuda.Stream() for _ in hs]
+    streams = [t.cuda.Stream(), t.cuda.default_stream() if default else t.cuda.Stream()]
     t.cuda.synchronize()
     for _ in range(4):
         for h in hs:

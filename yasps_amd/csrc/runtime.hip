@@ -139,36 +139,48 @@ std::mutex g_element_mutex;
 bool g_element_used = false;              // an evaluation was queued on g_element_stream
 hipStream_t g_element_stream = nullptr;
 hipEvent_t g_element_event = nullptr;
+bool g_element_recorded = false;          // the event is recorded behind the last evaluation
 
 bool capturing(hipStream_t s) {
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(s, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
 }
 
-// Makes s wait for what the last evaluation's stream holds (event recorded now).
+void record_elements(hipStream_t s) {
+  g_element_recorded =
+      (g_element_event ||
+       hipEventCreateWithFlags(&g_element_event, hipEventDisableTiming) == hipSuccess) &&
+      hipEventRecord(g_element_event, s) == hipSuccess;
+  if (!g_element_recorded) (void)hipGetLastError();
+}
+
 int order_elements(hipStream_t s) {
-  if (g_element_used && g_element_stream == s) return YSP_OK;
+  // hipStreamPerThread is another stream in every thread
+  if (g_element_used && g_element_stream == s && s != hipStreamPerThread) return YSP_OK;
   if (capturing(s)) return YSP_OK;
-  if (g_element_used && !capturing(g_element_stream)) {
-    if (!g_element_event)
-      YSP_CHECK(hipEventCreateWithFlags(&g_element_event, hipEventDisableTiming));
-    // a stream that was destroyed meanwhile cannot be waited for by itself
-    if (hipEventRecord(g_element_event, g_element_stream) != hipSuccess ||
-        hipStreamWaitEvent(s, g_element_event, 0) != hipSuccess) {
-      (void)hipGetLastError();
+  if (g_element_used && (g_element_recorded || !capturing(g_element_stream))) {
+    if (!g_element_recorded) record_elements(g_element_stream);
+    // a stream that was destroyed meanwhile takes no event
+    if (g_element_recorded)
+      YSP_CHECK(hipStreamWaitEvent(s, g_element_event, 0));
+    else
       YSP_CHECK(hipDeviceSynchronize());
-    }
   }
   g_element_used = true;
   g_element_stream = s;
+  g_element_recorded = false;
   return YSP_OK;
 }
 }  // namespace
 
 namespace ysp {
-ElementScratchOrder::ElementScratchOrder(hipStream_t s) {
+ElementScratchOrder::ElementScratchOrder(hipStream_t s) : stream_(s) {
   g_element_mutex.lock();
   rc = order_elements(s);
 }
-ElementScratchOrder::~ElementScratchOrder() { g_element_mutex.unlock(); }
+ElementScratchOrder::~ElementScratchOrder() {
+  // no other thread's call can name this thread's own stream
+  if (stream_ == hipStreamPerThread && rc == YSP_OK && !capturing(stream_)) record_elements(stream_);
+  g_element_mutex.unlock();
+}
 }  // namespace ysp
